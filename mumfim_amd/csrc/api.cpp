@@ -446,8 +446,9 @@ int make_plan(mf_batch *b, int prec) {
   return MF_OK;
 }
 
-// Tangent-linear variant of every RVE: the fewest threads, then the fewest
-// node slots per thread, that hold its free nodes and fit the LDS.
+// Tangent-linear variant of every RVE: three directions per workgroup where
+// its LDS holds them, then the fewest node slots per thread, then the fewest
+// threads, that hold its free nodes.
 void make_plan_tl(mf_batch *b) {
   int nv = 0;
   const Variant *vs = variants(&nv);
@@ -461,7 +462,7 @@ void make_plan_tl(mf_batch *b) {
       if (!(v.flags & kTangentLinear) || (long)v.block * v.npt < p.Nf) continue;
       const size_t L = lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries);
       if (L > kMaxLds) continue;
-      const long key = (long)v.npt * 100000 + v.block;
+      const long key = (tl_dirs(v.flags) > 1 ? 0L : 10000000L) + (long)v.npt * 100000 + v.block;
       if (b->plan_tl[r] < 0 || key < best_key) {
         b->plan_tl[r] = i;
         b->lds_tl[r] = L;
@@ -743,13 +744,20 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
   const std::vector<size_t> &plds = S.tl ? b->lds_tl : b->lds[prec];
   std::vector<int32_t> order(n);
   for (int i = 0; i < n; ++i) order[i] = i;
-  if (S.tl)  // grouped by variant, largest RVEs first
+  if (S.tl) {
+    // workgroups of one or several directions (the solves come six to an
+    // RVE, in direction order), named by their first; grouped by variant,
+    // largest RVEs first
+    int nvt = 0;
+    const Variant *vt = variants(&nvt);
+    order.clear();
+    for (int i = 0; i < n; i += tl_dirs(vt[plan[S.rve[i]]].flags)) order.push_back(i);
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
       const int vx = plan[S.rve[x]], vy = plan[S.rve[y]];
       if (vx != vy) return vx > vy;
       return b->host[S.rve[x]].M > b->host[S.rve[y]].M;
     });
-  else
+  } else
     order = launch_order(b, prec, n, [&](int i) { return S.rve[i]; });
   MF_HIP(hipMemcpyAsync(b->solve_rve.p, S.rve.data(), sizeof(int32_t) * n,
                         hipMemcpyHostToDevice, s));
@@ -757,7 +765,8 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
                         hipMemcpyHostToDevice, s));
   MF_HIP(hipMemcpyAsync(b->solve_F.p, S.F.data(), sizeof(double) * 9 * n,
                         hipMemcpyHostToDevice, s));
-  MF_HIP(hipMemcpyAsync(b->order.p, order.data(), sizeof(int32_t) * n,
+  const int nu = (int)order.size();  // workgroups
+  MF_HIP(hipMemcpyAsync(b->order.p, order.data(), sizeof(int32_t) * nu,
                         hipMemcpyHostToDevice, s));
   SolveArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -805,12 +814,12 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
   std::vector<int64_t> ggs;
   int nv = 0;
   const Variant *vs = variants(&nv);
-  for (int i = 0; i < n;) {
+  for (int i = 0; i < nu;) {
     int v = plan[S.rve[order[i]]];
     int j = i;
     size_t L = 0;
     int maxN = 0;
-    while (j < n && plan[S.rve[order[j]]] == v) {
+    while (j < nu && plan[S.rve[order[j]]] == v) {
       L = std::max(L, plds[S.rve[order[j]]]);
       maxN = std::max(maxN, b->host[S.rve[order[j]]].N);
       ++j;

@@ -207,6 +207,9 @@ static const Variant kVariants[] = {
 #define MF_TL_ENTRY(B, N) {MF_PREC_FP32C, B, N, kTangentLinear},
     MF_TL_LIST(MF_TL_ENTRY)
 #undef MF_TL_ENTRY
+#define MF_TLK_ENTRY(B, N) {MF_PREC_FP32C, B, N, kTangentLinear | (kTlDirs << kFplShift)},
+    MF_TLK_LIST(MF_TLK_ENTRY)
+#undef MF_TLK_ENTRY
 };
 
 const Variant *variants(int *count) {
@@ -228,6 +231,9 @@ size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries) {
   if (v.flags & kTangentLinear) {
     // displacements, their derivatives, reference coordinates; scratch;
     // boundary state (FP64) and its derivative (FP32); packed table
+    if (tl_dirs(v.flags) == kTlDirs)
+      return 64 * Np + sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nbp +
+             48 * Nbp + sizeof(float) * 4 * 3 * kMaxReactions;
     return 48 * Np + sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nbp +
            16 * Nbp + sizeof(float) * 4 * 3 * kMaxReactions;
   }

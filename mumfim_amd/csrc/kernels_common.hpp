@@ -327,6 +327,56 @@ __device__ inline float react32_mix2_d(const ReactDev &nl, float ea_half_lin, bo
   return is_nl ? (ext ? te : tt) : ea_half_lin * il * e2;
 }
 
+// react32_tab_d and react32_mix2_d with their contractions spelt out as the
+// one-direction kernel's compilation chose them, for kernels whose results
+// must be its bits.
+__device__ inline float react32_tab_dt(const float4 *T, unsigned rid, float e2, float il,
+                                       float &dt) {
+  const float4 a = T[kReactTabStride * rid];
+  const float4 b = T[kReactTabStride * rid + 1], c = T[kReactTabStride * rid + 2];
+  dt = a.x * il;
+  const float tl = dt * e2;
+  if (a.w == 0.0f) return tl;
+  const bool hi = e2 > b.x, lo = e2 < c.x;
+  const float x = a.z * fminf(fmaxf(e2, c.x), b.x);
+  float em;
+  if (fabsf(x) <= kToePolyMax) {
+    float p = fmaf(x, 1.0f / 5040.0f, 1.0f / 720.0f);
+    p = fmaf(x, p, 1.0f / 120.0f);
+    p = fmaf(x, p, 1.0f / 24.0f);
+    p = fmaf(x, p, 1.0f / 6.0f);
+    p = fmaf(x, p, 0.5f);
+    p = fmaf(x, p, 1.0f);
+    em = p * x;
+  } else {
+    em = __expf(x) - 1.0f;
+  }
+  const float tt = a.y * il * em;
+  const float ilam = __frsqrt_rn(1.0f + e2);
+  const float C = hi ? b.z : c.z;
+  const float te = ext_law(hi ? b.y : c.y, C, il, ilam);
+  const float dte = (0.5f * C * il) * (ilam * (ilam * ilam));
+  const bool ext = hi || lo;
+  dt = ext ? dte : a.z * fmaf(il, a.y, tt);
+  return ext ? te : tt;
+}
+__device__ inline float react32_mix2_dt(const ReactDev &nl, float ea_half_lin, bool is_nl,
+                                        float e2, float il, float &dt) {
+  const bool hi = e2 > nl.lt2m1, lo = e2 < nl.lc2m1;
+  float p = fmaf(nl.pe[6], e2, nl.pe[5]);
+#pragma unroll
+  for (int k = 4; k >= 0; --k) p = fmaf(e2, p, nl.pe[k]);
+  const float tt = il * (e2 * p);
+  const float ilam = __frsqrt_rn(1.0f + e2);
+  const float C = hi ? nl.Ct : nl.Cc;
+  const float te = ext_law(hi ? nl.Kt : nl.Kc, C, il, ilam);
+  const float dte = (0.5f * C * il) * (ilam * (ilam * ilam));
+  const bool ext = hi || lo;
+  const float dl = ea_half_lin * il;
+  dt = is_nl ? (ext ? dte : nl.B_half * fmaf(nl.alpha, il, tt)) : dl;
+  return is_nl ? (ext ? te : tt) : dl * e2;
+}
+
 // The reaction table qualifies for react32_mix2 (uniform over the
 // workgroup); nl_rid and ea_half_lin describe it.
 __device__ inline bool mix2_table(const ReactDev *q, int n, int &nl_rid, float &ea_half_lin) {
@@ -357,6 +407,9 @@ struct Lin64 {
 
 // Tangent-linear FP32c variants: (threads, free-node slots per thread).
 #define MF_TL_LIST(X) X(256, 1) X(512, 1) X(1024, 1) X(1024, 2) X(1024, 3)
+
+// The same with kTlDirs directions per workgroup.
+#define MF_TLK_LIST(X) X(256, 1) X(512, 1) X(768, 1) X(768, 2) X(768, 3)
 
 // Fiber-streamed FP32c variants (large RVEs): (threads, fibers per thread,
 // free nodes per thread, reaction mode flag kLinearOnly|kMix2).  The widest

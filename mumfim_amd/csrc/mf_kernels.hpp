@@ -104,6 +104,10 @@ constexpr int kWaveBufStride = 384;
 // other flags stay clear of them).
 constexpr int kFplShift = 8;
 inline int variant_fpl(int32_t flags) { return (flags >> kFplShift) & 15; }
+// Directions per workgroup of the tangent-linear variants that say so in the
+// same bits (the others take one); divides an RVE's six.
+constexpr int kTlDirs = 3;
+inline int tl_dirs(int32_t flags) { return variant_fpl(flags) ? variant_fpl(flags) : 1; }
 
 
 
