@@ -190,9 +190,12 @@ struct mf_batch {
   DevBuf<RveDev> rves;
   DevBuf<double> X, mass, l0, V, cur_stress, F_in;
   DevBuf<int32_t> deg, slice_base, slice_D, ell_w, fib, fstream, ell_fref;
-  DevBuf<double> ell_l0;
+  DevBuf<double> ell_l0, ell_r0;
+  DevBuf<uint32_t> fs_ab;
+  DevBuf<double2> fs_lr;
   DevBuf<float> ell_il, fparam;
   DevBuf<ReactDev> reacts;
+  DevBuf<Law64> laws;
   DevBuf<double> xs[2], us[2];
   int cur = 0;
   bool have_run = false;   // current_stress_ valid
@@ -326,7 +329,7 @@ bool variant_fits(const mf_batch *b, int prec, const Variant &v, const PackedRVE
   if (v.flags & kTangentLinear) return false;
   if (v.flags & kGlobalState)  // FP64, any size; also the FP32c fallback
     return !(prec == MF_PREC_FP64 && b->p.energy_diagnostics) && block_ok(b, prec, v) &&
-           lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries) <= kMaxLds;
+           lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries, p.t_records) <= kMaxLds;
   if (v.prec != prec) return false;
   if (!block_ok(b, prec, v)) return false;
   const bool regs = (v.flags & kEllInRegs) != 0;
@@ -338,6 +341,11 @@ bool variant_fits(const mf_batch *b, int prec, const Variant &v, const PackedRVE
     return false;
   if ((v.flags & kLinearOnly) && !lin) return false;
   if ((v.flags & kMix2) && !mix2_ok(p)) return false;
+  if ((v.flags & kFast64) && (!p.fast64 || p.max_free_deg > 255)) return false;
+  if ((v.flags & kFiberOnce) && !(v.flags & kFast64) &&
+      (!p.fast64 || ((v.flags & kLinearOnly) && !p.one_linear) ||
+       (long)v.block * fonce_fpl(v) < p.M))
+    return false;
   if (((v.flags & kEnergy) != 0) != (prec == MF_PREC_FP64 && b->p.energy_diagnostics != 0))
     return false;
   if (regs && b->no_reg_variants) return false;
@@ -351,7 +359,7 @@ bool variant_fits(const mf_batch *b, int prec, const Variant &v, const PackedRVE
     return false;
   // one RVE per wave: a workgroup holds block / 64 regions of this size
   const size_t regions = wave ? (size_t)v.block / 64 : 1;
-  return regions * ((lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries) + 15) & ~size_t(15)) <=
+  return regions * ((lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries, p.t_records) + 15) & ~size_t(15)) <=
          kMaxLds;
 }
 
@@ -420,8 +428,11 @@ int make_plan(mf_batch *b, int prec) {
       // ones, whose cheap force does not pay for the extra phase (13% slower
       // on 500-node RVEs)
       long key = (v.flags & kGlobalState) ? 2000000000L
+                 : (v.flags & kFast64)
+                     ? ((v.flags & kFiberOnce) ? 600000000L : 700000000L) +
+                           (long)v.npt * 10000000 + (long)v.block * 1000
                  : (v.flags & kFiberOnce)
-                     ? (lin ? 1500000000L : 500000000L) + (long)v.npt * 10000000 + (long)v.block * 1000
+                     ? 500000000L + (long)v.npt * 10000000 + (long)v.block * 1000 + mode_rank
                  : fpar ? (lin ? 50000000L : 15000000L) + fpl * 100000 + (long)v.block * 10 + mode_rank
                  : fstr ? (lin ? 55000000L : 15350000L) + (v.block > 768 ? 50000L : 0L) +
                               (long)v.npt * 10000 + fpl * 100 + mode_rank
@@ -441,7 +452,7 @@ int make_plan(mf_batch *b, int prec) {
       return MF_ERR_UNSUPPORTED;
     }
     b->plan[prec][r] = best;
-    b->lds[prec][r] = lds_bytes(vs[best], p.N, p.Nb, p.M, p.ell_free_entries);
+    b->lds[prec][r] = lds_bytes(vs[best], p.N, p.Nb, p.M, p.ell_free_entries, p.t_records);
   }
   return MF_OK;
 }
@@ -460,7 +471,7 @@ void make_plan_tl(mf_batch *b) {
     for (int i = 0; i < nv; ++i) {
       const Variant &v = vs[i];
       if (!(v.flags & kTangentLinear) || (long)v.block * v.npt < p.Nf) continue;
-      const size_t L = lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries);
+      const size_t L = lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries, p.t_records);
       if (L > kMaxLds) continue;
       const long key = (tl_dirs(v.flags) > 1 ? 0L : 10000000L) + (long)v.npt * 100000 + v.block;
       if (b->plan_tl[r] < 0 || key < best_key) {
@@ -496,9 +507,9 @@ int upload_batch(mf_batch *b) {
     d.n_slices = (int)p.slice_base.size();
     d.ell_free_entries = p.ell_free_entries;
     d.n_split = p.n_split;
-    d.m_free = 0;
-    for (int e = 0; e < p.M; ++e)
-      if (p.fstream[4 * (size_t)e + 2] >= 0) d.m_free = e + 1;
+    d.m_free = p.m_free;
+    d.n_nl = p.n_nl;
+    d.t_records = p.t_records;
     d.react_off = (int)rx.size();
     d.n_react = (int)p.reactions.size();
     d.c_sound = p.c_sound;
@@ -545,12 +556,20 @@ int upload_batch(mf_batch *b) {
   MF_HIP(b->slice_D.upload(sD, s));
   MF_HIP(b->ell_w.upload(ew, s));
   MF_HIP(b->ell_l0.upload(ell_l0, s));
+  MF_HIP(b->ell_r0.alloc(ell_l0.size()));
+  MF_HIP(launch_reciprocal(b->ell_l0.p, b->ell_r0.p, (int64_t)ell_l0.size(), s));
   MF_HIP(b->ell_il.upload(il, s));
   MF_HIP(b->fib.upload(fib, s));
   MF_HIP(b->fstream.upload(fst, s));
   MF_HIP(b->ell_fref.upload(efr, s));
+  MF_HIP(b->fs_ab.alloc((size_t)fib_off));
+  MF_HIP(b->fs_lr.alloc((size_t)fib_off));
+  MF_HIP(launch_stream64(b->rves.p, R, b->fstream.p, b->ell_w.p, b->ell_l0.p, b->fs_ab.p,
+                         b->fs_lr.p, s));
   MF_HIP(b->fparam.upload(fpm, s));
   MF_HIP(b->reacts.upload(rx, s));
+  MF_HIP(b->laws.alloc(rx.size()));
+  MF_HIP(launch_laws(b->reacts.p, b->laws.p, (int)rx.size(), s));
   // state: x = X, u = 0, V = 1 (constructor, ...Explicit.h:115-118,250-253)
   for (int k = 0; k < 2; ++k) {
     MF_HIP(b->xs[k].upload(X, s));
@@ -778,12 +797,16 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
   a.slice_D = b->slice_D.p;
   a.ell_w = b->ell_w.p;
   a.ell_l0 = b->ell_l0.p;
+  a.ell_r0 = b->ell_r0.p;
+  a.fs_ab = b->fs_ab.p;
+  a.fs_lr = b->fs_lr.p;
   a.ell_il = b->ell_il.p;
   a.fib = b->fib.p;
   a.fstream = b->fstream.p;
   a.ell_fref = b->ell_fref.p;
   a.fparam = b->fparam.p;
   a.reacts = b->reacts.p;
+  a.laws = b->laws.p;
   a.x_in = x_in;
   a.u_in = u_in;
   a.x_out = x_out;
@@ -842,12 +865,16 @@ void fill_args(mf_batch *b, SolveArgs &a) {
   a.slice_D = b->slice_D.p;
   a.ell_w = b->ell_w.p;
   a.ell_l0 = b->ell_l0.p;
+  a.ell_r0 = b->ell_r0.p;
+  a.fs_ab = b->fs_ab.p;
+  a.fs_lr = b->fs_lr.p;
   a.ell_il = b->ell_il.p;
   a.fib = b->fib.p;
   a.fstream = b->fstream.p;
   a.ell_fref = b->ell_fref.p;
   a.fparam = b->fparam.p;
   a.reacts = b->reacts.p;
+  a.laws = b->laws.p;
   a.V = b->V.p;
   a.steps = b->steps.p;
   a.mode = b->p.mode;
@@ -1613,7 +1640,7 @@ int mf_batch_autotune(mf_batch *b, int32_t precision, int32_t steps, const char 
         for (int r : L) {
           b->plan[prec][r] = i;
           b->lds[prec][r] = lds_bytes(vs[i], b->host[r].N, b->host[r].Nb, b->host[r].M,
-                                      b->host[r].ell_free_entries);
+                                      b->host[r].ell_free_entries, b->host[r].t_records);
         }
         const int cidx = b->cur;
         double us = 0.0;

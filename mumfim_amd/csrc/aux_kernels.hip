@@ -98,6 +98,32 @@ __global__ void fd_column_kernel(const double *sig1, const double *sig0,
         (sig1[(int64_t)r * s1 + j] - sig0[(int64_t)r * s0 + j]) / h;
 }
 
+// Fiber-stream words, reference lengths and their reciprocals (one workgroup
+// per RVE).
+__global__ void stream64_kernel(const RveDev *rves, const int32_t *fstream, const int32_t *ell_w,
+                                const double *ell_l0, uint32_t *ab, double2 *lr) {
+  const RveDev R = rves[blockIdx.x];
+  for (int e = threadIdx.x; e < R.M; e += blockDim.x) {
+    const int32_t *q = fstream + 4 * (R.fib_off + e);
+    const int sa = q[2];
+    const uint32_t rid = sa >= 0 ? (uint32_t)ell_w[R.ell_off + sa] >> 24 : 0;
+    const double l0 = sa >= 0 ? ell_l0[R.ell_off + sa] : 1.0;
+    ab[R.fib_off + e] = ((uint32_t)q[0] & 0x3FFFu) | ((uint32_t)q[1] & 0x3FFFu) << 14 | rid << 28;
+    lr[R.fib_off + e] = make_double2(l0, 1.0 / l0);
+  }
+}
+
+// out[i] = 1 / in[i]
+__global__ void reciprocal_kernel(const double *in, double *out, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = 1.0 / in[i];
+}
+
+__global__ void laws_kernel(const ReactDev *reacts, Law64 *laws, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) laws[i] = make_law64(reacts[i]);
+}
+
 // Orientation tensors (BatchedComputeOrientationTensor.h:56-176), one
 // workgroup per RVE, FP64 block reduction.
 template <int B>
@@ -195,12 +221,16 @@ static const Variant kVariants[] = {
     MF_FIBER_STREAM_LIST(MF_FSTR_ENTRY)
 #undef MF_FSTR_ENTRY
     // FP64, each fiber evaluated once per step: (threads, free nodes per thread)
-    {MF_PREC_FP64, 256, 1, kFiberOnce},
-    {MF_PREC_FP64, 256, 2, kFiberOnce},
-    {MF_PREC_FP64, 512, 1, kFiberOnce},
-    {MF_PREC_FP64, 512, 2, kFiberOnce},
-    {MF_PREC_FP64, 1024, 1, kFiberOnce},
-    {MF_PREC_FP64, 1024, 2, kFiberOnce},
+#define MF_FONCE_ENTRY(B, N, FPL) \
+  {MF_PREC_FP64, B, N, kFiberOnce | kLinearOnly}, {MF_PREC_FP64, B, N, kFiberOnce},
+    MF_FONCE_LIST(MF_FONCE_ENTRY)
+#undef MF_FONCE_ENTRY
+#define MF_NODE64_ENTRY(B, N) {MF_PREC_FP64, B, N, kFast64},
+    MF_NODE64_LIST(MF_NODE64_ENTRY)
+#undef MF_NODE64_ENTRY
+#define MF_FONCE_L_ENTRY(B, N) {MF_PREC_FP64, B, N, kFiberOnce | kFast64},
+    MF_NODE64_LIST(MF_FONCE_L_ENTRY)
+#undef MF_FONCE_L_ENTRY
     // FP64 with the state in global memory: RVEs no other variant holds
     {MF_PREC_FP64, 1024, 1, kGlobalState},
     // FP32c tangent-linear: (threads, free nodes per thread)
@@ -217,16 +247,26 @@ const Variant *variants(int *count) {
   return kVariants;
 }
 
-size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries) {
+int fonce_fpl(const Variant &v) {
+#define MF_FONCE_FPL(B, N, FPL) \
+  if (v.block == B && v.npt == N) return FPL;
+  MF_FONCE_LIST(MF_FONCE_FPL)
+#undef MF_FONCE_FPL
+  return 0;
+}
+
+size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries, int t_records) {
   const size_t Np = (N + 1) & ~1, Nbp = (Nb + 1) & ~1;
   const size_t NW = (v.flags & kWaveRve) ? 1 : v.block / kern::kWave;  // waves per RVE
   size_t b = 0;
+  if (v.flags & kFast64)  // positions, t records, scratch, boundary state
+    return 24 * Np + ((v.flags & kFiberOnce) ? 8 * (((size_t)t_records + 1) & ~size_t(1)) : 0) +
+           sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nb;
   if (v.flags & kFiberOnce) {
-    // double-buffered positions, t per fiber (M bounds the fibers with a
-    // free end), scratch, boundary state, reactions
-    return sizeof(double) * 6 * Np + sizeof(double) * (((size_t)M + 1) & ~size_t(1)) +
-           sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nbp +
-           ((sizeof(ReactDev) * kMaxReactions + 15) & ~size_t(15));
+    // positions, a force record per fiber (M bounds the fibers with a free
+    // end) and a zero record, scratch, boundary state
+    b = 24 * (Np + (((size_t)M + 2) & ~size_t(1)));
+    return b + sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nb;
   }
   if (v.flags & kTangentLinear) {
     // displacements, their derivatives, reference coordinates; scratch;
@@ -240,7 +280,7 @@ size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries) {
   if (v.flags & kGlobalState) {
     // scratch, boundary state, reactions (positions etc. in global memory)
     return sizeof(double) * NW * kern::kRedStride + sizeof(double) * 6 * Nbp +
-           ((sizeof(ReactDev) * kMaxReactions + 15) & ~size_t(15));
+           ((sizeof(Law64) * kMaxReactions + 15) & ~size_t(15));
   }
   if (v.flags & kFiberStream) {
     // 12-byte displacement and force records (+ zero record), scratch,
@@ -268,7 +308,7 @@ size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries) {
   b += sizeof(double) * NW * kern::kRedStride;
   b += sizeof(double) * 6 * Nbp;
   if (v.flags & kEnergy) b += sizeof(double) * 3 * Nbp;
-  b += v.prec == MF_PREC_FP64 ? (sizeof(ReactDev) * kMaxReactions + 15) & ~size_t(15)
+  b += v.prec == MF_PREC_FP64 ? (sizeof(Law64) * kMaxReactions + 15) & ~size_t(15)
                               : sizeof(float) * 4 * 3 * kMaxReactions;  // packed table
   if (v.flags & kEllInLds)
     b += (size_t)ell_free_entries *
@@ -289,6 +329,28 @@ hipError_t launch_solve(const Variant &v, const SolveArgs &a, int n_blocks,
   if (v.flags & kTangentLinear) return launch_solve32t(v, a, n_blocks, lds, s);
   return v.prec == MF_PREC_FP64 ? launch_solve64(v, a, n_blocks, lds, s)
                                 : launch_solve32(v, a, n_blocks, lds, s);
+}
+
+hipError_t launch_laws(const ReactDev *reacts, Law64 *laws, int n, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(kern::laws_kernel, dim3((n + 255) / 256), dim3(256), 0, s, reacts, laws, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_stream64(const RveDev *rves, int n_rve, const int32_t *fstream,
+                           const int32_t *ell_w, const double *ell_l0, uint32_t *ab, double2 *lr,
+                           hipStream_t s) {
+  if (n_rve <= 0) return hipSuccess;
+  hipLaunchKernelGGL(kern::stream64_kernel, dim3(n_rve), dim3(256), 0, s, rves, fstream, ell_w,
+                     ell_l0, ab, lr);
+  return hipGetLastError();
+}
+
+hipError_t launch_reciprocal(const double *in, double *out, int64_t n, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(kern::reciprocal_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                     in, out, n);
+  return hipGetLastError();
 }
 
 hipError_t lds_probe(double *bytes_per_s) {

@@ -74,10 +74,12 @@ __device__ inline void block_sum(double (&v)[NV], double *red) {
 // Ramp-mode boundary amplitude after step k (1-based) of S:
 // linear xi = k/S, or SmoothAmp xi^3 (10 - 15 xi + 6 xi^2)
 // (ExplicitAmplitude.h:26-40), evaluated in the reference's operation order.
-__device__ inline double ramp_alpha(int k, int S, int amplitude) {
-  const double xi = (double)k / (double)S;
+__device__ inline double amplitude64(double xi, int amplitude) {
   if (amplitude == MF_AMP_SMOOTHSTEP) return xi * xi * xi * (10 - 15 * xi + 6 * xi * xi);
   return xi;
+}
+__device__ inline double ramp_alpha(int k, int S, int amplitude) {
+  return amplitude64((double)k / (double)S, amplitude);
 }
 
 
@@ -159,36 +161,42 @@ __device__ inline int4 ld16(const int4 *p) {
   return make_int4(v.x, v.y, v.z, v.w);
 }
 
+// Fiber-stream words of the large-RVE FP64 kernel (fs_ab): both ranks (14 bits
+// each) and the reaction id.
+__device__ inline uint32_t stream_a(uint32_t q) { return q & 0x3FFFu; }
+__device__ inline uint32_t stream_b(uint32_t q) { return q >> 14 & 0x3FFFu; }
+__device__ inline int stream_law(uint32_t q) { return (int)(q >> 28); }
+
 // ---- reaction laws, FP64 reference formulas (FiberReactions.cc:5-71) ------
-__device__ inline double nl_force(double alpha, double B, double lr,
-                                  double g) {
-  return alpha * lr * (exp(B * g) - 1);
-}
-__device__ inline double nl_deriv(double alpha, double B, double lr, double l0,
-                                  double g) {
-  return alpha / l0 * ((1 + lr * lr * B) * exp(B * g) - 1);
-}
-__device__ inline double react64(const ReactDev &q, double l0, double l) {
+__device__ inline Law64 make_law64(const ReactDev &q) {
 #pragma clang fp contract(off)
-  double lr = l / l0;
-  if (q.type == MF_REACTION_LINEAR) {
-    double g = 1.0 / 2.0 * (lr * lr - 1);
-    return lr * q.E * q.A * g;
-  }
-  double alpha = q.E * q.A / q.B;
-  if (lr > q.lt) {
-    double gt = 1.0 / 2.0 * (q.lt * q.lt - 1);
-    double m = nl_deriv(alpha, q.B, q.lt, l0, gt);
-    double b = nl_force(alpha, q.B, q.lt, gt);
-    return m * (lr - q.lt) * l0 + b;
-  } else if (lr < q.lc) {
-    double gc = 1.0 / 2.0 * (q.lc * q.lc - 1);
-    double m = nl_deriv(alpha, q.B, q.lc, l0, gc);
-    double b = nl_force(alpha, q.B, q.lc, gc);
-    return m * (lr - q.lc) * l0 + b;
-  }
-  double g = 1.0 / 2.0 * (lr * lr - 1);
-  return nl_force(alpha, q.B, lr, g);
+  Law64 w;
+  w.E = q.E;
+  w.A = q.A;
+  w.B = q.B;
+  w.lt = q.lt;
+  w.lc = q.lc;
+  w.type = q.type;
+  w.pad_ = 0;
+  w.alpha = w.Kt = w.bt = w.Kc = w.bc = 0.0;
+  if (q.type == MF_REACTION_LINEAR) return w;
+  w.alpha = q.E * q.A / q.B;
+  const double et = exp(q.B * (1.0 / 2.0 * (q.lt * q.lt - 1)));
+  const double ec = exp(q.B * (1.0 / 2.0 * (q.lc * q.lc - 1)));
+  w.Kt = (1 + q.lt * q.lt * q.B) * et - 1;
+  w.bt = w.alpha * q.lt * (et - 1);
+  w.Kc = (1 + q.lc * q.lc * q.B) * ec - 1;
+  w.bc = w.alpha * q.lc * (ec - 1);
+  return w;
+}
+__device__ inline double react64(const Law64 &q, double l0, double l) {
+#pragma clang fp contract(off)
+  const double lr = l / l0;
+  const double g = 1.0 / 2.0 * (lr * lr - 1);
+  if (q.type == MF_REACTION_LINEAR) return lr * q.E * q.A * g;
+  if (lr > q.lt) return q.alpha / l0 * q.Kt * (lr - q.lt) * l0 + q.bt;
+  if (lr < q.lc) return q.alpha / l0 * q.Kc * (lr - q.lc) * l0 + q.bc;
+  return q.alpha * lr * (exp(q.B * g) - 1);
 }
 
 // ---- reaction laws, FP32 algebraic forms --------------------------------
@@ -443,6 +451,16 @@ struct Lin64 {
   X(1024, 2, 1, kLinearOnly) X(1024, 2, 1, kMix2)                            \
   X(1024, 3, 2, kLinearOnly) X(1024, 3, 2, kMix2)                            \
   X(1024, 4, 2, kLinearOnly) X(1024, 4, 2, kMix2)
+
+// Fiber-once FP64 variants: (threads, free-node slots per thread, fibers per
+// thread held in registers), each for RVEs of one linear reaction and for any
+// reaction table.  k = 4 neighbour networks have ~2.8 fibers per free node.
+#define MF_FONCE_LIST(X)                                                     \
+  X(256, 1, 3) X(256, 2, 6) X(512, 1, 3) X(512, 2, 6) X(1024, 1, 3) X(1024, 2, 5)
+
+// FP64 variants for fast64 RVEs whose force records do not fit LDS, with t
+// records and node-centric: (threads, free-node slots per thread).
+#define MF_NODE64_LIST(X) X(1024, 2) X(1024, 3) X(1024, 4)
 
 // Compiled kernel variants: (precision, threads, free-node slots per thread,
 // flags kEllInLds|kDoubleBuf).

@@ -108,6 +108,14 @@ struct PackedRVE {
   std::vector<double> l0;              // M
   std::vector<int32_t> rid;            // M (after the reaction policy)
   std::vector<Reaction> reactions;     // after the reaction policy
+  // FP64: lengths, masses and stiffnesses lie so far inside the range that
+  // square roots and quotients need no scaling (2^-300 to 2^300)
+  bool fast64 = false;
+  // fibers with a free end, and the nonlinear ones among them where both laws
+  // occur (they come first in the stream; else 0); records of the large-RVE
+  // FP64 kernel, which takes the two laws one after the other
+  int m_free = 0, n_nl = 0, t_records = 0;
+  bool one_linear = false;  // every fiber: a linear reaction with reaction 0's E and radius
   double scale = 1.0;
   double c_sound = 0.0;                // sqrt(E/rho) used for the time step
   // Mean fiber length, fiber density, nonlinear fraction (surrogate inputs).
@@ -128,6 +136,8 @@ struct RveDev {
   int32_t react_off;
   int32_t n_react;
   int32_t m_free;     // fibers with a free end (the fiber-stream prefix)
+  int32_t n_nl;       // nonlinear ones among them, first, where both laws occur
+  int32_t t_records;
   double c_sound, scale;
   // Reference coordinates in fixed point for the FP32 kernel: X_q =
   // rint(X * xq_scale) fits int32; xq_scale is a power of two.
@@ -158,6 +168,19 @@ struct ReactDev {
   // alpha (B/2)^k / k!, k = 1..7 (the Taylor polynomial with both scalings
   // folded in)
   float pe[7];
+};
+
+// A reaction for the FP64 kernels, with what does not depend on the fiber
+// formed once per batch: alpha = E A / B, and for an extension beyond a
+// transition L the factor K = (1 + L^2 B) exp(B g) - 1 of its slope
+// alpha / l0 K and its value b = alpha L (exp(B g) - 1) there
+// (FiberReactions.cc:16-71).  The operations and their order are the
+// reference's, so the forces keep its bits; evaluated per fiber and step, each
+// of a wave's two extension branches took two exponentials and two divisions.
+struct Law64 {
+  double E, A, alpha, B, lt, lc;
+  double Kt, bt, Kc, bc;
+  int32_t type, pad_;
 };
 
 }  // namespace mf

@@ -21,12 +21,16 @@ struct SolveArgs {
   const int32_t *slice_base, *slice_D;
   const int32_t *ell_w;
   const double *ell_l0;     // FP64 kernels
+  const double *ell_r0;     // 1 / ell_l0
+  const uint32_t *fs_ab;    // fiber stream: ranks and reaction in one word
+  const double2 *fs_lr;     // fiber stream: l0, 1 / l0
   const float *ell_il;      // FP32 kernels: 1/l0
   const int32_t *fib;       // 2 per fiber (kernel ranks)
   const int32_t *fstream;   // 4 per fiber: ranks a, b and their ELL entries
   const int32_t *ell_fref;  // per ELL entry: fiber record index | sign bit
   const float *fparam;      // 4 per fiber: reference vector, law coefficient
   const ReactDev *reacts;
+  const Law64 *laws;        // FP64 laws of the same reactions
   const double *x_in, *u_in;
   double *x_out, *u_out;
   const double *V;          // per RVE
@@ -90,7 +94,10 @@ enum : int32_t {
   kFiberStream = 128,  // FP32c fiber-streamed: per-fiber forces, nodes gather by reference
   kWaveRve = 4096,     // FP32c registers, one RVE per wave, block / 64 RVEs per workgroup
   kGlobalState = 8192, // FP64 state in global memory: any RVE size
-  kFiberOnce = 16384,  // FP64, t = f/l once per fiber, nodes gather by reference
+  kFiberOnce = 16384,  // FP64, d t once per fiber, nodes gather by reference
+  // FP64 for fast64 RVEs whose force records do not fit LDS: t records with
+  // kFiberOnce, node-centric without
+  kFast64 = 65536,
   kTangentLinear = 32768,  // FP32c solve with its derivative along solve_G
 };
 // Stride (float4 entries) of the two position buffers of the register
@@ -121,7 +128,10 @@ struct Variant {
 // All compiled variants (the planner picks from this list).
 const Variant *variants(int *count);
 // LDS bytes a variant needs for one RVE (N nodes, Nb boundary, M fibers).
-size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries);
+// t_records: records of the large-RVE FP64 kernel (PackedRVE).
+size_t lds_bytes(const Variant &v, int N, int Nb, int M, int ell_free_entries, int t_records);
+// Fibers per thread a fiber-once FP64 variant holds in registers.
+int fonce_fpl(const Variant &v);
 // Largest dynamic LDS a workgroup may request.
 constexpr size_t kMaxLds = 160 * 1024;
 
@@ -132,6 +142,14 @@ hipError_t launch_solve(const Variant &v, const SolveArgs &a, int n_blocks,
 int chunk_occupancy(const Variant &v, size_t lds);
 hipError_t lds_probe(double *bytes_per_s);
 hipError_t hbm_probe(int64_t bytes, double *bytes_per_s);
+// laws[i] = the FP64 law of reacts[i] (once per batch).
+hipError_t launch_laws(const ReactDev *reacts, Law64 *laws, int n, hipStream_t s);
+// fs_ab and fs_lr of every fiber.
+hipError_t launch_stream64(const RveDev *rves, int n_rve, const int32_t *fstream,
+                           const int32_t *ell_w, const double *ell_l0, uint32_t *ab, double2 *lr,
+                           hipStream_t s);
+// out[i] = 1 / in[i].
+hipError_t launch_reciprocal(const double *in, double *out, int64_t n, hipStream_t s);
 hipError_t launch_broadcast_F(const double *F, double *out, int n, hipStream_t s);
 hipError_t launch_update_volume(const double *F, int nF, double *V, int n_rve,
                                 hipStream_t s);

@@ -414,6 +414,16 @@ int pack_rve(const Network &net, int reaction_policy, PackedRVE &p) {
     p.mass[p.fib[2 * e]] += c;
     p.mass[p.fib[2 * e + 1]] += c;
   }
+  auto mid_range = [](double v) { return v >= 0x1p-300 && v <= 0x1p300; };
+  p.fast64 = true;
+  p.one_linear = p.reactions[0].type == MF_REACTION_LINEAR;
+  for (int e = 0; e < M; ++e) {
+    const Reaction &r = p.reactions[p.rid[e]];
+    p.fast64 = p.fast64 && mid_range(p.l0[e]) && mid_range(r.E) && mid_range(r.area());
+    p.one_linear = p.one_linear && r.type == MF_REACTION_LINEAR &&
+                   r.E == p.reactions[0].E && r.radius == p.reactions[0].radius;
+  }
+  for (int r = 0; r < p.Nf; ++r) p.fast64 = p.fast64 && mid_range(p.mass[r]);
   p.max_free_deg = 0;
   p.n_split = 0;
   for (int r = 0; r < p.Nf; ++r) {
@@ -518,6 +528,15 @@ int pack_rve(const Network &net, int reaction_policy, PackedRVE &p) {
       }
     p.fstream.swap(part);
   }
+  p.m_free = (int)(p.fstream.size() / 4);
+  p.n_nl = 0;
+  if (mixed)
+    while (p.n_nl < p.m_free &&
+           p.reactions[(uint32_t)p.ell_w[p.fstream[4 * (size_t)p.n_nl + 2]] >> 24].type ==
+               MF_REACTION_NONLINEAR)
+      ++p.n_nl;
+  if (p.n_nl == p.m_free) p.n_nl = 0;
+  p.t_records = std::max(p.n_nl, p.m_free - p.n_nl);
   for (int e = 0; e < M; ++e)
     if (!taken[e]) p.fstream.insert(p.fstream.end(), {p.fib[2 * e], p.fib[2 * e + 1], -1, -1});
   p.fparam.assign(4 * (size_t)M, 0.0f);
