@@ -48,6 +48,14 @@ constexpr int kTRows = 272;  // transposed hidden activations: 256 + ones row + 
 constexpr int64_t kW1 = kHid * kInP, kW2 = kHid * kHid, kW4 = kOutP * kHid;
 constexpr int64_t kW4T = kHid * kInP;
 constexpr int64_t kBias = 3 * kHid + kOutP;
+// Position of element (row, k) of a BF16 operand of padded width kp kept in
+// fragment order: the 16 rows x 32 k that one MFMA reads are one contiguous
+// kilobyte, lane after lane, so a fragment load touches 8 whole 128-byte
+// lines (row by row it touches 16 half lines).
+__host__ __device__ constexpr int64_t frag(int64_t row, int64_t k, int64_t kp) {
+  return ((row >> 4) * (kp >> 5) + (k >> 5)) * 512 + (((k & 31) >> 3) * 16 + (row & 15)) * 8 +
+         (k & 7);
+}
 constexpr int kActLd = kHid + 8;  // LDS row stride (BF16) of the inference tile
 
 __device__ __forceinline__ uint16_t bf(float x) {
@@ -153,12 +161,16 @@ __global__ __launch_bounds__(256) void gemm_nt(GemmArgs g) {
   const int64_t k0 = (int64_t)split * g.kc + lk;
   const uint16_t *pa0 = g.A + mem * g.sA + (int64_t)(r0 + lr) * g.lda + k0;
   const uint16_t *pa1 = row1 ? pa0 + 16 * g.lda : pa0;
-  const uint16_t *pb0 = g.B + mem * g.sB + (int64_t)(c0 + lr) * g.ldb + k0;
+  // weights are in fragment order
+  constexpr bool FB = EPI != kPartial;
+  const uint16_t *pb0 = g.B + mem * g.sB + (FB ? frag(c0, 0, g.ldb) + lane * 8
+                                               : (int64_t)(c0 + lr) * g.ldb + k0);
   const uint16_t *pb1 = col1 ? pb0 + 16 * g.ldb : pb0;
+  constexpr int kb = FB ? 16 : 1;
   f32x4 a00 = {0.f, 0.f, 0.f, 0.f}, a01 = a00, a10 = a00, a11 = a00;
   for (int k = 0; k < g.kc; k += 32) {
     const bf16x8 x0 = ld8(pa0 + k), x1 = ld8(pa1 + k);
-    const bf16x8 y0 = ld8(pb0 + k), y1 = ld8(pb1 + k);
+    const bf16x8 y0 = ld8(pb0 + kb * k), y1 = ld8(pb1 + kb * k);
     a00 = mfma(x0, y0, a00);
     a01 = mfma(x0, y1, a01);
     a10 = mfma(x1, y0, a10);
@@ -292,18 +304,18 @@ __global__ void adam_kernel(AdamArgs a) {
     return;
   }
   switch (L) {
-    case 0: a.w1[mem * kW1 + o * kInP + i] = u; break;
+    case 0: a.w1[mem * kW1 + frag(o, i, kInP)] = u; break;
     case 1:
-      a.w2[mem * kW2 + o * kHid + i] = u;
-      a.w2t[mem * kW2 + i * kHid + o] = u;
+      a.w2[mem * kW2 + frag(o, i, kHid)] = u;
+      a.w2t[mem * kW2 + frag(i, o, kHid)] = u;
       break;
     case 2:
-      a.w3[mem * kW2 + o * kHid + i] = u;
-      a.w3t[mem * kW2 + i * kHid + o] = u;
+      a.w3[mem * kW2 + frag(o, i, kHid)] = u;
+      a.w3t[mem * kW2 + frag(i, o, kHid)] = u;
       break;
     default:
-      a.w4[mem * kW4 + o * kHid + i] = u;
-      a.w4t[mem * kW4T + i * kInP + o] = u;
+      a.w4[mem * kW4 + frag(o, i, kHid)] = u;
+      a.w4t[mem * kW4T + frag(i, o, kInP)] = u;
       break;
   }
 }
@@ -316,14 +328,25 @@ __global__ void ones_row_kernel(uint16_t *T, int64_t member_stride, int one_row,
 }
 
 // ---------------------------------------------------------------------------
-// Fused inference.  A tile holds TS = 16 Q samples; with JAC it also holds
-// six tangent planes (d/d e_j of every activation), so the LDS tile has
-// P = Q * planes blocks of 16 rows, one row per (plane, sample), 256 BF16
-// features per row.  Each layer computes the transposed product
-// W (features) x act^T (rows): wave w owns features [64w, 64w + 64) and lane
-// l ends up with 4 consecutive features of one row, written back as one
+// Fused inference.  A tile holds TS = 16 Q samples; with NT > 0 it also holds
+// NT of the six tangent planes (d/d e_j of every activation; blockIdx.y picks
+// which), so the LDS tile has P = Q (1 + NT) blocks of 16 rows, one row per
+// (plane, sample), 256 BF16 features per row.  Each layer computes the
+// transposed product W (features) x act^T (rows): a wave owns 32 features and
+// lane l ends up with 4 consecutive features of one row, written back as one
 // 8-byte LDS store.  Plane 0 takes bias and silu, plane j the product with
-// silu'(z) of the same (sample, feature), which sits in the same lane.
+// silu'(z) of the same (sample, feature), which sits in the same lane.  G
+// members are evaluated at a time, eight waves each, and added in order.
+//
+// What bounds it: the activations' VALU work (2^20 samples, four members:
+// 1.0 ms of 1.4 ms) and, with J, the matrix cores (0.55 ms) and the weights'
+// way through L2 (280 KB per tile and member).  Measured on 2^20 samples /
+// 150001 with J: 2.73 / 2.31 ms with weights row by row, four waves of 64
+// features and accumulators in AGPRs (two or three waves per SIMD, each value
+// copied back before use); 2.39 / 1.49 ms with eight waves of 32 features (four
+// waves per SIMD, no copies, weights one k step ahead); 1.39 / 1.03 ms with
+// the weights in fragment order (row by row, a fragment is 16 half lines and
+// the vector cache's line rate was the bound).
 struct InferArgs {
   const float *X;
   int64_t n;
@@ -334,35 +357,57 @@ struct InferArgs {
   float *Y, *J, *spread;
 };
 
-template <int P, int KS>
-__device__ __forceinline__ void infer_layer(const uint16_t *act, const uint16_t *W, int ldw,
-                                            int w, int lr, int lk, f32x4 (&acc)[P][4]) {
+// A wave's weight fragments of one k step: its 16 C features x 32 k.
+template <int C>
+struct WFrag {
+  bf16x8 v[C];
+};
+template <int C, int KP>
+__device__ __forceinline__ WFrag<C> load_w(const uint16_t *W, int kk, int w, int lane) {
+  // uniform base (w is a scalar) plus one 32-bit lane offset for all blocks
+  const uint32_t off = (uint32_t)lane * 16u;
+  WFrag<C> f;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    f.v[c] = *reinterpret_cast<const bf16x8 *>(
+        reinterpret_cast<const char *>(W + ((C * w + c) * (KP / 32) + kk) * 512) + off);
+  return f;
+}
+
+// acc = W (16 C features of wave w) x act^T (16 P rows) over KS k steps.  `wf`
+// holds the first step's weights (loaded before the barrier that published
+// act); each later step's load while the one before is multiplied.
+template <int P, int C, int KS, int LDA>
+__device__ __forceinline__ void infer_layer(const uint16_t *act, const uint16_t *W, int w, int lane,
+                                            WFrag<C> wf, f32x4 (&acc)[P][C]) {
 #pragma unroll
   for (int p = 0; p < P; ++p)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[p][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < C; ++c) acc[p][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
-    bf16x8 wa[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) wa[c] = ld8(W + (64 * w + 16 * c + lr) * ldw + 32 * kk + lk);
+    WFrag<C> nx;
+    if (kk + 1 < KS) nx = load_w<C, 32 * KS>(W, kk + 1, w, lane);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const bf16x8 x = ld8(act + (16 * p + lr) * kActLd + 32 * kk + lk);
+      const bf16x8 x = ld8(act + (16 * p + (lane & 15)) * LDA + 32 * kk + (lane >> 4) * 8);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[p][c] = mfma(wa[c], x, acc[p][c]);
+      for (int c = 0; c < C; ++c) acc[p][c] = mfma(wf.v[c], x, acc[p][c]);
     }
+    // with all seven planes the loads of several steps at once would spill
+    if (P > 4) __builtin_amdgcn_sched_barrier(0);
+    if (kk + 1 < KS) wf = nx;
   }
 }
 
-template <int Q, int NPL>
-__device__ __forceinline__ void infer_hidden_epilogue(uint16_t *act, f32x4 (&acc)[Q * NPL][4],
-                                                      const float *bias, int w, int lr,
+template <int Q, int NPL, int C>
+__device__ __forceinline__ void infer_hidden_epilogue(uint16_t *act, f32x4 (&acc)[Q * NPL][C],
+                                                      const float4 (&bias)[C], int w, int lr,
                                                       int lq) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int f0 = 64 * w + 16 * c + lq;
-    const float4 b = *reinterpret_cast<const float4 *>(bias + f0);
+  for (int c = 0; c < C; ++c) {
+    const int f0 = 16 * (C * w + c) + lq;
+    const float4 b = bias[c];
 #pragma unroll
     for (int sb = 0; sb < Q; ++sb) {
       float h[4], d[4];
@@ -383,97 +428,141 @@ __device__ __forceinline__ void infer_hidden_epilogue(uint16_t *act, f32x4 (&acc
   }
 }
 
-template <int Q, bool JAC>
-__global__ __launch_bounds__(256) void infer_kernel(InferArgs a) {
-  constexpr int NPL = JAC ? 7 : 1;
+template <int C>
+__device__ __forceinline__ void load_bias(const float *bias, int w, int lq, float4 (&b)[C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    b[c] = *reinterpret_cast<const float4 *>(
+        reinterpret_cast<const char *>(bias + 16 * (C * w + c)) + (uint32_t)lq * 4u);
+}
+
+constexpr int kInferWaves = 8;  // waves that evaluate one member of a tile
+constexpr int kInLd = kInP + 8;  // LDS row stride (BF16) of the input tile
+constexpr int kOutLd = 8;        // LDS row stride (FP32) of a member's outputs
+// LDS of an inference workgroup of P row blocks and G members at a time: the
+// input tile, each member's activations and (G > 1) its outputs.
+constexpr size_t infer_lds(int P, int G) {
+  return (size_t)P * 16 *
+         ((kInLd + G * kActLd) * sizeof(uint16_t) + (G - 1) * kOutLd * sizeof(float));
+}
+
+template <int Q, int NT, int G>
+__global__ __launch_bounds__(64 * kInferWaves * G, 4) void infer_kernel(InferArgs a) {
+  constexpr int NW = kInferWaves, NPL = 1 + NT;
   constexpr int P = Q * NPL;
   constexpr int TS = 16 * Q;
-  constexpr int OWN = (P + 3) / 4;
-  extern __shared__ uint16_t act[];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int lr = lane & 15, lk = (lane >> 4) * 8, lq = (lane >> 4) * 4;
+  static_assert(P <= NW, "one output block per wave");
+  constexpr int C = 16 / NW;  // 16-feature blocks per wave
+  extern __shared__ uint16_t lds[];
+  uint16_t *const xin = lds;
+  const int tid = threadIdx.x;
+  const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wg % NW, grp = wg / NW;  // wave of its member, member group
+  uint16_t *const act = lds + P * 16 * (kInLd + grp * kActLd);
+  float *const osh = reinterpret_cast<float *>(lds + P * 16 * (kInLd + G * kActLd));
+  const int j0 = NT ? NT * blockIdx.y : 0;  // first tangent direction
   const int64_t s0 = (int64_t)blockIdx.x * TS;
   const MlpNorm *nm = a.nm;
-  f32x4 fsum[OWN], fsq[OWN];
-#pragma unroll
-  for (int t = 0; t < OWN; ++t) fsum[t] = fsq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[P][4];
-  for (int mi = 0; mi < a.mcount; ++mi) {
-    const int mem = a.m0 + mi;
-    // inputs: plane 0 = normalised x (10 of 32 columns), plane j = e_j seed
-    for (int e = tid; e < P * 16 * kInP; e += 256) {
-      const int row = e / kInP, c = e % kInP;
-      const int plane = row / TS, sr = row % TS;
-      float v = 0.f;
-      if (plane == 0) {
-        const int64_t s = s0 + sr;
-        if (c < kIn && s < a.n) v = (a.X[s * kIn + c] - nm->in_mean[c]) * nm->in_inv[c];
-      } else if (c == plane - 1) {
-        v = 1.f;
-      }
-      act[row * kActLd + c] = bf(v);
+  // inputs, the same for every member: plane 0 = normalised x (10 of 32
+  // columns), plane j = e_j seed
+  for (int e = tid; e < P * 16 * kInP; e += 64 * NW * G) {
+    const int row = e / kInP, c = e % kInP;
+    const int plane = row / TS, sr = row % TS;
+    float v = 0.f;
+    if (plane == 0) {
+      const int64_t s = s0 + sr;
+      if (c < kIn && s < a.n) v = (a.X[s * kIn + c] - nm->in_mean[c]) * nm->in_inv[c];
+    } else if (c == j0 + plane - 1) {
+      v = 1.f;
     }
-    __syncthreads();
-    const float *bias = a.bias + mem * kBias;
-    infer_layer<P, 1>(act, a.w1 + mem * kW1, kInP, w, lr, lk, acc);
-    __syncthreads();
-    infer_hidden_epilogue<Q, NPL>(act, acc, bias, w, lr, lq);
-    __syncthreads();
-    infer_layer<P, 8>(act, a.w2 + mem * kW2, kHid, w, lr, lk, acc);
-    __syncthreads();
-    infer_hidden_epilogue<Q, NPL>(act, acc, bias + kHid, w, lr, lq);
-    __syncthreads();
-    infer_layer<P, 8>(act, a.w3 + mem * kW2, kHid, w, lr, lk, acc);
-    __syncthreads();
-    infer_hidden_epilogue<Q, NPL>(act, acc, bias + 2 * kHid, w, lr, lq);
-    __syncthreads();
-    // output layer: 16 (6 used) features x 16 rows per block, blocks
-    // w, w + 4, ... owned by wave w
-    const uint16_t *W4 = a.w4 + mem * kW4;
-    const float4 b4 = *reinterpret_cast<const float4 *>(bias + 3 * kHid + lq);
-#pragma unroll
-    for (int t = 0; t < OWN; ++t) {
-      const int p = w + 4 * t;
-      if (p < P) {
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-          o = mfma(ld8(W4 + lr * kHid + 32 * kk + lk),
-                   ld8(act + (16 * p + lr) * kActLd + 32 * kk + lk), o);
-        if (p < Q) {
-          o[0] += b4.x;
-          o[1] += b4.y;
-          o[2] += b4.z;
-          o[3] += b4.w;
-          fsq[t] += o * o;
-        }
-        fsum[t] += o;
-      }
-    }
-    __syncthreads();
+    xin[row * kInLd + c] = bf(v);
   }
-  const float inv_m = 1.0f / (float)a.mcount;
+  f32x4 fsum = {0.f, 0.f, 0.f, 0.f}, fsq = fsum;
+  f32x4 acc[P][C];
+  const int last = a.m0 + a.mcount - 1;
+  int mem = min(a.m0 + grp, last);
+  WFrag<C> wf = load_w<C, kInP>(a.w1 + mem * kW1, 0, w, tid & 63);
+  __syncthreads();
+#pragma clang loop unroll(disable)
+  for (int m = a.m0; m <= last; m += G) {
+    // a group without a member of its own repeats the last one, unread
+    mem = min(m + grp, last);
+    // the lane's offsets are worked out anew: kept over the loop they spill
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
+    const int lr = lane & 15, lq = (lane >> 4) * 4;
+    const float *bias = a.bias + mem * kBias;
+    const uint16_t *W2 = a.w2 + mem * kW2, *W3 = a.w3 + mem * kW2, *W4 = a.w4 + mem * kW4;
+    // before each epilogue the next product's first weights are requested:
+    // they arrive while the activations are evaluated
+    float4 b[C];
+    load_bias<C>(bias, w, lq, b);
+    infer_layer<P, C, 1, kInLd>(xin, a.w1 + mem * kW1, w, lane, wf, acc);
+    wf = load_w<C, kHid>(W2, 0, w, lane);
+    __syncthreads();  // the last member's output products have read act
+    infer_hidden_epilogue<Q, NPL, C>(act, acc, b, w, lr, lq);
+    __syncthreads();
+    load_bias<C>(bias + kHid, w, lq, b);
+    infer_layer<P, C, 8, kActLd>(act, W2, w, lane, wf, acc);
+    wf = load_w<C, kHid>(W3, 0, w, lane);
+    __syncthreads();
+    infer_hidden_epilogue<Q, NPL, C>(act, acc, b, w, lr, lq);
+    __syncthreads();
+    load_bias<C>(bias + 2 * kHid, w, lq, b);
+    infer_layer<P, C, 8, kActLd>(act, W3, w, lane, wf, acc);
+    __syncthreads();
+    infer_hidden_epilogue<Q, NPL, C>(act, acc, b, w, lr, lq);
+    if (m + G <= last) wf = load_w<C, kInP>(a.w1 + min(m + G + grp, last) * kW1, 0, w, lane);
+    const float4 b4 = *reinterpret_cast<const float4 *>(bias + 3 * kHid + lq);
+    __syncthreads();
+    // output layer: 16 (6 used) features x 16 rows, row block w by wave w
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    if (w < P) {
 #pragma unroll
-  for (int t = 0; t < OWN; ++t) {
-    const int p = w + 4 * t;
-    if (p >= P) continue;
-    const int plane = p / Q, sb = p % Q;
-    const int64_t s = s0 + 16 * sb + lr;
-    if (s >= a.n) continue;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = lq + q;
-      if (i >= kOut) continue;
-      const float mean = fsum[t][q] * inv_m;
-      if (plane == 0) {
-        a.Y[s * kOut + i] = mean * nm->out_std[i] + nm->out_mean[i];
-        if (a.spread) {
-          const float var = fmaxf(fsq[t][q] * inv_m - mean * mean, 0.f);
-          a.spread[s * kOut + i] = sqrtf(var) * nm->out_std[i];
+      for (int kk = 0; kk < 8; ++kk)
+        o = mfma(load_w<1, kHid>(W4, kk, 0, lane).v[0],
+                 ld8(act + (16 * w + lr) * kActLd + 32 * kk + (lane >> 4) * 8), o);
+      if (w < Q) o += f32x4{b4.x, b4.y, b4.z, b4.w};
+    }
+    if (G == 1) {
+      if (w < Q) fsq += o * o;
+      fsum += o;
+    } else {  // group 0 adds the outputs in member order
+      float4 *const row = reinterpret_cast<float4 *>(osh + (16 * w + lr) * kOutLd + lq);
+      const bool mine = w < P && lq < kOutLd;
+      if (grp == 1 && mine) *row = make_float4(o[0], o[1], o[2], o[3]);
+      __syncthreads();
+      if (grp == 0 && mine) {
+        fsq += o * o;
+        fsum += o;
+        if (m < last) {
+          const float4 r = *row;
+          const f32x4 o1 = {r.x, r.y, r.z, r.w};
+          fsq += o1 * o1;
+          fsum += o1;
         }
-      } else {
-        a.J[s * 36 + 6 * i + (plane - 1)] = mean * nm->out_std[i] * nm->in_inv[plane - 1];
       }
+    }
+  }
+  if (grp > 0 || w >= P) return;
+  const float inv_m = 1.0f / (float)a.mcount;
+  const int plane = w / Q, lr = tid & 15, lq = ((tid & 63) >> 4) * 4;
+  const int64_t s = s0 + 16 * (w % Q) + lr;
+  if (s >= a.n || (plane == 0 && blockIdx.y > 0)) return;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int i = lq + q;
+    if (i >= kOut) continue;
+    const float mean = fsum[q] * inv_m;
+    if (plane == 0) {
+      a.Y[s * kOut + i] = mean * nm->out_std[i] + nm->out_mean[i];
+      if (a.spread) {
+        const float var = fmaxf(fsq[q] * inv_m - mean * mean, 0.f);
+        a.spread[s * kOut + i] = sqrtf(var) * nm->out_std[i];
+      }
+    } else {
+      const int j = j0 + plane - 1;
+      a.J[s * 36 + 6 * i + j] = mean * nm->out_std[i] * nm->in_inv[j];
     }
   }
 }
@@ -797,6 +886,20 @@ int forward_backward(mf_mlp *m, const float *X, const float *Y, int64_t n_data,
   return MF_OK;
 }
 
+constexpr int kCus = 256;  // compute units of the chip
+template <int Q, int NT, int G>
+void launch_infer(const InferArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL((infer_kernel<Q, NT, G>),
+                     dim3((unsigned)((a.n + 16 * Q - 1) / (16 * Q)), NT ? 6 / NT : 1),
+                     dim3(64 * kInferWaves * G), infer_lds(Q * (1 + NT), G), s, a);
+}
+template <int Q, int NT, int G>
+hipError_t infer_attr() {
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(&infer_kernel<Q, NT, G>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)infer_lds(Q * (1 + NT), G));
+}
+
 bool valid_batch(int64_t Bt) { return Bt > 0 && Bt % MF_MLP_BATCH_ALIGN == 0 && Bt <= (1 << 24); }
 
 }  // namespace
@@ -823,16 +926,22 @@ int mlp_predict(mf_mlp *m, int member, const float *X, int64_t n, float *Y, floa
   a.Y = Y;
   a.J = J;
   a.spread = spread;
+  // Up to one workgroup per CU the time is the chain of layers and members, so
+  // the call is cut finer: two members at a time, 16 samples and (with J) two
+  // of the six tangent planes per workgroup, each repeating plane 0.  Four
+  // members, wide against fine: 777 points with J 47 -> 33 us (1361 points,
+  // two workgroups on some CUs: 47 against 48), 4096 points without J
+  // 42 -> 29.5 us (5600 points: 42 against 42).
+  const int64_t t16 = (n + 15) / 16;
   if (J) {
-    constexpr int Q = 1, P = 7;
-    const size_t lds = (size_t)P * 16 * kActLd * sizeof(uint16_t);
-    hipLaunchKernelGGL((infer_kernel<Q, true>), dim3((unsigned)((n + 16 * Q - 1) / (16 * Q))),
-                       dim3(256), lds, s, a);
+    if (3 * t16 <= kCus)
+      launch_infer<1, 2, 2>(a, s);
+    else
+      launch_infer<1, 6, 1>(a, s);
+  } else if (t16 <= kCus) {
+    launch_infer<1, 0, 2>(a, s);
   } else {
-    constexpr int Q = 4, P = 4;
-    const size_t lds = (size_t)P * 16 * kActLd * sizeof(uint16_t);
-    hipLaunchKernelGGL((infer_kernel<Q, false>), dim3((unsigned)((n + 16 * Q - 1) / (16 * Q))),
-                       dim3(256), lds, s, a);
+    launch_infer<4, 0, 1>(a, s);
   }
   MF_HIP(hipGetLastError());
   return MF_OK;
@@ -905,12 +1014,8 @@ int mf_mlp_create(int32_t n_members, uint64_t seed, mf_mlp **out) {
   }
   static bool attr_done = false;
   if (!attr_done) {
-    const int big = 4 * 16 * kActLd * (int)sizeof(uint16_t);
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&infer_kernel<4, false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, big) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void *>(&infer_kernel<1, true>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            7 * 16 * kActLd * (int)sizeof(uint16_t)) != hipSuccess) {
+    if (infer_attr<4, 0, 1>() != hipSuccess || infer_attr<1, 0, 2>() != hipSuccess ||
+        infer_attr<1, 6, 1>() != hipSuccess || infer_attr<1, 2, 2>() != hipSuccess) {
       set_error("mf_mlp_create: LDS attribute");
       return fail(MF_ERR_HIP);
     }
