@@ -9,13 +9,11 @@
 // rows 4*(l >> 4) .. 4*(l >> 4) + 3 of column (l & 15).  Every operand here
 // is stored with k contiguous, so each lane's fragment is one 16-byte load.
 //
-// Training (one launch per layer and pass, all members in grid.z):
-//   prep       gather the mini-batch, normalise, round to BF16
-//   fwd 1..4   Z = A W^T + b; hidden layers store H = silu(Z), H^T and
-//              silu'(Z) (BF16); the output layer stores Y (FP32)
-//   loss       dL/dY of the mean squared error (BF16, both layouts)
-//   bwd 4..2   D = (D_next W) * silu'(Z)  (W^T copies as the B operand)
-//   dW 1..4    D^T H over the batch, split over K into FP32 partials; the
+// Training, three launches per mini-batch, all members in each:
+//   train      per tile of samples, in LDS and registers: gather, normalise,
+//              the four layers, the loss, the gradients back to layer 1;
+//              leaves the transposed activations and gradients (BF16)
+//   dw         D^T H over the batch, split over K into FP32 partials; the
 //              transposed activations carry a row of ones, so the bias
 //              gradient is one more column of the same product
 //   adam       sums the partials in a fixed order (deterministic), updates
@@ -56,6 +54,7 @@ __host__ __device__ constexpr int64_t frag(int64_t row, int64_t k, int64_t kp) {
   return ((row >> 4) * (kp >> 5) + (k >> 5)) * 512 + (((k & 31) >> 3) * 16 + (row & 15)) * 8 +
          (k & 7);
 }
+constexpr int kCus = 256;           // compute units of the chip
 constexpr int kActLd = kHid + 8;  // LDS row stride (BF16) of the inference tile
 
 __device__ __forceinline__ uint16_t bf(float x) {
@@ -89,167 +88,38 @@ __device__ __forceinline__ bf16x8 ld8(const uint16_t *p) {
 }
 
 // ---------------------------------------------------------------------------
-// Generic C = A B^T (A: M x K, B: N x K, both BF16 with K contiguous).  Each
-// wave computes one 32 x 32 tile (2 x 2 MFMA tiles); grid.y splits K,
-// grid.z is the ensemble member.  M and N are multiples of 16, kc of 32.
-enum Epi { kFwdHidden = 0, kFwdOut = 1, kBwdHidden = 2, kPartial = 3 };
-
-struct GemmArgs {
-  const uint16_t *A, *B;
-  int64_t lda, ldb, sA, sB;
-  int M, N, kc;
-  const float *bias;
-  int64_t sbias;
-  const uint16_t *Sin;  // silu'(Z) of the layer below (kBwdHidden), ld ldo
-  uint16_t *O, *OT, *OS;
-  int64_t ldo, ldt, sO, sOT;
-  float *Y;
-  int64_t ldy, sY, sYsplit;
-};
-
-template <int EPI>
-__device__ __forceinline__ void gemm_store(const GemmArgs &g, f32x4 v, int rb, int cb,
-                                           int mem, int split, int lane) {
-  const int col = cb + (lane & 15);
-  const int row = rb + (lane >> 4) * 4;  // rows row .. row + 3
-  if constexpr (EPI == kPartial) {
-    float *Y = g.Y + mem * g.sY + split * g.sYsplit + col;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) Y[(int64_t)(row + q) * g.ldy] = v[q];
-  } else if constexpr (EPI == kFwdOut) {
-    const float b = g.bias[mem * g.sbias + col];
-    float *Y = g.Y + mem * g.sY + col;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) Y[(int64_t)(row + q) * g.ldy] = v[q] + b;
-  } else if constexpr (EPI == kFwdHidden) {
-    const float b = g.bias[mem * g.sbias + col];
-    float h[4], d[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) h[q] = silu(v[q] + b, d[q]);
-    uint16_t *O = g.O + mem * g.sO + col, *S = g.OS + mem * g.sO + col;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      O[(int64_t)(row + q) * g.ldo] = bf(h[q]);
-      S[(int64_t)(row + q) * g.ldo] = bf(d[q]);
-    }
-    *reinterpret_cast<uint2 *>(g.OT + mem * g.sOT + (int64_t)col * g.ldt + row) =
-        pack4(h[0], h[1], h[2], h[3]);
-  } else {  // kBwdHidden
-    const uint16_t *S = g.Sin + mem * g.sO + col;
-    float d[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) d[q] = v[q] * unbf(S[(int64_t)(row + q) * g.ldo]);
-    uint16_t *O = g.O + mem * g.sO + col;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) O[(int64_t)(row + q) * g.ldo] = bf(d[q]);
-    *reinterpret_cast<uint2 *>(g.OT + mem * g.sOT + (int64_t)col * g.ldt + row) =
-        pack4(d[0], d[1], d[2], d[3]);
-  }
-}
-
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm_nt(GemmArgs g) {
-  const int lane = threadIdx.x & 63;
-  const int tiles_n = (g.N + 31) >> 5;
-  const int tiles = ((g.M + 31) >> 5) * tiles_n;
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= tiles) return;  // whole wave; the kernel has no barriers
-  const int r0 = (tile / tiles_n) * 32, c0 = (tile % tiles_n) * 32;
-  const bool row1 = r0 + 16 < g.M, col1 = c0 + 16 < g.N;
-  const int mem = blockIdx.z, split = blockIdx.y;
-  const int lr = lane & 15, lk = (lane >> 4) * 8;
-  const int64_t k0 = (int64_t)split * g.kc + lk;
-  const uint16_t *pa0 = g.A + mem * g.sA + (int64_t)(r0 + lr) * g.lda + k0;
-  const uint16_t *pa1 = row1 ? pa0 + 16 * g.lda : pa0;
-  // weights are in fragment order
-  constexpr bool FB = EPI != kPartial;
-  const uint16_t *pb0 = g.B + mem * g.sB + (FB ? frag(c0, 0, g.ldb) + lane * 8
-                                               : (int64_t)(c0 + lr) * g.ldb + k0);
-  const uint16_t *pb1 = col1 ? pb0 + 16 * g.ldb : pb0;
-  constexpr int kb = FB ? 16 : 1;
-  f32x4 a00 = {0.f, 0.f, 0.f, 0.f}, a01 = a00, a10 = a00, a11 = a00;
-  for (int k = 0; k < g.kc; k += 32) {
-    const bf16x8 x0 = ld8(pa0 + k), x1 = ld8(pa1 + k);
-    const bf16x8 y0 = ld8(pb0 + kb * k), y1 = ld8(pb1 + kb * k);
-    a00 = mfma(x0, y0, a00);
-    a01 = mfma(x0, y1, a01);
-    a10 = mfma(x1, y0, a10);
-    a11 = mfma(x1, y1, a11);
-  }
-  gemm_store<EPI>(g, a00, r0, c0, mem, split, lane);
-  if (col1) gemm_store<EPI>(g, a01, r0, c0 + 16, mem, split, lane);
-  if (row1) {
-    gemm_store<EPI>(g, a10, r0 + 16, c0, mem, split, lane);
-    if (col1) gemm_store<EPI>(g, a11, r0 + 16, c0 + 16, mem, split, lane);
-  }
-}
-
-// Gathers member k's mini-batch rows idx[k*idx_stride + b], normalises them
-// and writes the BF16 inputs in both layouts plus the FP32 targets.
-__global__ void prep_kernel(const float *X, const float *Y, int64_t n_data,
-                            const int32_t *idx, int64_t idx_stride, int Bt,
-                            const MlpNorm *nm, uint16_t *Xn, uint16_t *XnT,
-                            float *Yt) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  const int mem = blockIdx.y;
-  if (b >= Bt) return;
-  int64_t r = idx ? idx[mem * idx_stride + b] : b;
-  r = r < 0 ? 0 : (r >= n_data ? n_data - 1 : r);
-  uint16_t *xn = Xn + (int64_t)mem * Bt * kInP + (int64_t)b * kInP;
-  uint16_t *xt = XnT + (int64_t)mem * kInP * Bt + b;
-  for (int i = 0; i < kIn; ++i) {
-    const uint16_t u = bf((X[r * kIn + i] - nm->in_mean[i]) * nm->in_inv[i]);
-    xn[i] = u;
-    xt[(int64_t)i * Bt] = u;
-  }
-  float *yt = Yt + (int64_t)mem * Bt * 8 + (int64_t)b * 8;
-  for (int i = 0; i < kOut; ++i) yt[i] = (Y[r * kOut + i] - nm->out_mean[i]) * nm->out_inv[i];
-}
-
-__device__ float block_sum256(float v, float *red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
-}
-
-// Mean squared error of the normalised outputs and dL/dY = 2 (y - t)/(6 Bt).
-__global__ __launch_bounds__(256) void loss_kernel(const float *Yo, const float *Yt,
-                                                   int Bt, float gscale, uint16_t *D4,
-                                                   uint16_t *D4T, float *loss_part,
-                                                   int nblk) {
-  __shared__ float red[4];
-  const int b = blockIdx.x * 256 + threadIdx.x, mem = blockIdx.y;
-  float acc = 0.f;
-  if (b < Bt) {
-    const float *yo = Yo + (int64_t)mem * Bt * kOutP + (int64_t)b * kOutP;
-    const float *yt = Yt + (int64_t)mem * Bt * 8 + (int64_t)b * 8;
-    uint16_t *d = D4 + (int64_t)mem * Bt * kInP + (int64_t)b * kInP;
-    uint16_t *dt = D4T + (int64_t)mem * kOutP * Bt + b;
-    for (int i = 0; i < kOut; ++i) {
-      const float r = yo[i] - yt[i];
-      acc += r * r;
-      const uint16_t u = bf(r * gscale);
-      d[i] = u;
-      dt[(int64_t)i * Bt] = u;
-    }
-  }
-  const float s = block_sum256(acc, red);
-  if (threadIdx.x == 0) loss_part[mem * nblk + blockIdx.x] = s;
-}
-
-// Sums loss partials in block order (deterministic) into acc[mem] (+=) and
-// out[mem] (=).
-__global__ void loss_sum_kernel(const float *loss_part, int nblk, float inv,
-                                float *out, float *acc) {
-  const int mem = threadIdx.x;
-  if (mem >= (int)blockDim.x) return;
+// Loss of one member from its samples' squared errors: sums of 256 samples
+// (64 by a butterfly, four of those in order), added in batch order; out[mem]
+// = mean, acc[mem] += mean.
+__device__ void loss_sum(const float *v, int Bt, float inv, float *out, float *acc) {
+  constexpr int kGroups = 64;  // 64-sample groups per pass
+  __shared__ float red[kGroups];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   float s = 0.f;
-  for (int i = 0; i < nblk; ++i) s += loss_part[mem * nblk + i];
-  s *= inv;
-  out[mem] = s;
-  acc[mem] += s;
+  for (int64_t c = 0; c < Bt; c += 64 * kGroups) {
+    float x[kGroups / 4];
+#pragma unroll
+    for (int j = 0; j < kGroups / 4; ++j) {
+      const int64_t b = c + 64 * (w + 4 * j) + lane;
+      x[j] = b < Bt ? v[b] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < kGroups / 4; ++j) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) x[j] += __shfl_xor(x[j], o);
+      if (lane == 0) red[w + 4 * j] = x[j];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int g = 0; g < kGroups && c + 64 * g < Bt; g += 4)
+        s += red[g] + red[g + 1] + red[g + 2] + red[g + 3];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    s *= inv;
+    *out = s;
+    *acc += s;
+  }
 }
 
 struct AdamArgs {
@@ -263,13 +133,23 @@ struct AdamArgs {
   float lr, b1, b2, eps, bc1, bc2;
   float *grad;
   int mode;  // 0: Adam update, 1: gradient only, 2: refresh BF16 copies only
+  // the last block of each member sums the loss, where it is asked for
+  const float *loss_v;
+  int Bt;
+  float loss_inv, *loss_out, *loss_acc;
 };
 
 // One thread per (member, parameter): gradient = sum of the K-split
 // partials of its (layer, out, in) entry, in split order.
-__global__ void adam_kernel(AdamArgs a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int kAdamBlocks = (kNumParams + 255) / 256;
+__global__ __launch_bounds__(256) void adam_kernel(AdamArgs a) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
   const int mem = blockIdx.y;
+  if (blockIdx.x == kAdamBlocks) {
+    loss_sum(a.loss_v + (int64_t)mem * a.Bt, a.Bt, a.loss_inv, a.loss_out + mem,
+             a.loss_acc + mem);
+    return;
+  }
   if (p >= kNumParams) return;
   int L, o, i;
   bool isb = false;
@@ -286,7 +166,15 @@ __global__ void adam_kernel(AdamArgs a) {
   if (a.mode != 2) {
     const float *part = a.part[L] + mem * a.sPart[L] + (int64_t)o * a.ldp[L] + i;
     float g = 0.f;
-    for (int s = 0; s < a.splits; ++s) g += part[s * a.sSplit[L]];
+    int s = 0;
+    for (; s + 8 <= a.splits; s += 8) {  // eight loads in flight
+      float q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = part[(s + u) * a.sSplit[L]];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) g += q[u];
+    }
+    for (; s < a.splits; ++s) g += part[s * a.sSplit[L]];
     if (a.mode == 1) {
       a.grad[pi] = g;
       return;
@@ -320,11 +208,11 @@ __global__ void adam_kernel(AdamArgs a) {
   }
 }
 
-// Constant rows of the transposed activation buffers: row `one_row` of
+// Constant row of the transposed activation buffers: row `one_row` of
 // every member's [rows x Bt] block is 1.
 __global__ void ones_row_kernel(uint16_t *T, int64_t member_stride, int one_row, int Bt) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < Bt) T[blockIdx.y * member_stride + (int64_t)one_row * Bt + b] = bf(1.0f);
+  if (b < Bt) T[blockIdx.y * member_stride + frag(one_row, b, Bt)] = bf(1.0f);
 }
 
 // ---------------------------------------------------------------------------
@@ -568,6 +456,307 @@ __global__ __launch_bounds__(64 * kInferWaves * G, 4) void infer_kernel(InferArg
 }
 
 // ---------------------------------------------------------------------------
+// Training.  One workgroup takes 16 Q samples of one member through the
+// network and back, as in inference with the activations in LDS and a wave's
+// 32 features in registers; silu' of a layer stays in the registers of the
+// lanes that need it on the way back.  The operands of the weight gradients
+// (k = the batch) are read from the LDS tile feature by feature and written
+// as whole fragments.
+//
+// What bounds it, four members of 4096 samples: the chain of eight products
+// with one workgroup per CU, and 50 MB of operands written (25 us at 2 TB/s).
+// One product per launch, each in 32 x 32 tiles from and to memory in both
+// layouts, this took ten launches and 103 us.
+struct TrainArgs {
+  const float *X, *Y;
+  int64_t n_data;
+  const int32_t *idx;
+  int64_t idx_stride;
+  int Bt;
+  float gscale;  // 2 / (6 Bt)
+  const uint16_t *w1, *w2, *w3, *w4, *w2t, *w3t, *w4t;
+  const float *bias;
+  const MlpNorm *nm;
+  uint16_t *xt, *ht[3], *dt[3], *d4t;
+  float *loss_v;
+};
+
+// Row blocks [0, NB) of the transposed tile (its columns) to T in fragment
+// order: 32 samples x 16 columns per fragment, shared out over the waves.
+template <int Q, int NB>
+__device__ __forceinline__ void store_t(const uint16_t *tile, int ld, uint16_t *T, int Bt,
+                                        int64_t b0, int w, int lane) {
+  constexpr int KB = Q / 2;
+#pragma unroll
+  for (int i0 = 0; i0 < NB * KB; i0 += kInferWaves) {
+    const int i = i0 + w;
+    if (i >= NB * KB) break;
+    const int rb = i / KB, kb = i % KB;
+    const uint16_t *src = tile + (32 * kb + 8 * (lane >> 4)) * ld + 16 * rb + (lane & 15);
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] = (uint32_t)src[2 * j * ld] | (uint32_t)src[(2 * j + 1) * ld] << 16;
+    *reinterpret_cast<uint4 *>(T + frag(16 * rb, b0 + 32 * kb, Bt) + lane * 8) =
+        make_uint4(v[0], v[1], v[2], v[3]);
+  }
+}
+
+// act = silu(acc + bias), sd = silu' (BF16 pairs)
+template <int P, int C>
+__device__ __forceinline__ void train_epilogue(uint16_t *act, f32x4 (&acc)[P][C],
+                                               const float4 (&bias)[C], int w, int lr, int lq,
+                                               uint2 (&sd)[P][C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int f0 = 16 * (C * w + c) + lq;
+    const float4 b = bias[c];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      float h[4], d[4];
+      h[0] = silu(acc[p][c][0] + b.x, d[0]);
+      h[1] = silu(acc[p][c][1] + b.y, d[1]);
+      h[2] = silu(acc[p][c][2] + b.z, d[2]);
+      h[3] = silu(acc[p][c][3] + b.w, d[3]);
+      *reinterpret_cast<uint2 *>(act + (16 * p + lr) * kActLd + f0) =
+          pack4(h[0], h[1], h[2], h[3]);
+      sd[p][c] = pack4(d[0], d[1], d[2], d[3]);
+    }
+  }
+}
+
+// act = acc * silu'
+template <int P, int C>
+__device__ __forceinline__ void back_epilogue(uint16_t *act, f32x4 (&acc)[P][C], int w, int lr,
+                                              int lq, const uint2 (&sd)[P][C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int f0 = 16 * (C * w + c) + lq;
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+      *reinterpret_cast<uint2 *>(act + (16 * p + lr) * kActLd + f0) =
+          pack4(acc[p][c][0] * unbf(sd[p][c].x & 0xffff),
+                acc[p][c][1] * __uint_as_float(sd[p][c].x & 0xffff0000u),
+                acc[p][c][2] * unbf(sd[p][c].y & 0xffff),
+                acc[p][c][3] * __uint_as_float(sd[p][c].y & 0xffff0000u));
+  }
+}
+
+constexpr size_t train_lds(int P) {
+  return (size_t)P * 16 * (kActLd + 2 * kInLd) * sizeof(uint16_t);
+}
+
+template <int Q>
+__global__ __launch_bounds__(64 * kInferWaves, 2) void train_kernel(TrainArgs a) {
+  constexpr int P = Q, TS = 16 * Q, NW = kInferWaves, C = 16 / NW;
+  static_assert(Q % 2 == 0 && Q <= NW, "whole fragments of 32 samples, one output block a wave");
+  extern __shared__ uint16_t lds[];
+  uint16_t *const xin = lds, *const d4 = lds + TS * kInLd, *const act = lds + 2 * TS * kInLd;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = (lane >> 4) * 4;
+  const int64_t b0 = (int64_t)blockIdx.x * TS;
+  const int mem = blockIdx.y;
+  const MlpNorm *nm = a.nm;
+  const int32_t *idx = a.idx ? a.idx + mem * a.idx_stride + b0 : nullptr;
+  const auto row_of = [&](int b) {
+    const int64_t r = idx ? idx[b] : b0 + b;
+    return r < 0 ? 0 : (r >= a.n_data ? a.n_data - 1 : r);
+  };
+  for (int e = tid; e < TS * kInP; e += 64 * NW) {
+    const int b = e / kInP, c = e % kInP;
+    float v = 0.f;
+    if (c < kIn) v = (a.X[row_of(b) * kIn + c] - nm->in_mean[c]) * nm->in_inv[c];
+    xin[b * kInLd + c] = bf(v);
+    d4[b * kInLd + c] = 0;
+  }
+  float yt[4] = {0.f, 0.f, 0.f, 0.f};  // this lane's normalised targets
+  if (w < Q && lq < 8) {
+    const float *y = a.Y + row_of(16 * w + lr) * kOut;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (lq + q < kOut) yt[q] = (y[lq + q] - nm->out_mean[lq + q]) * nm->out_inv[lq + q];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(yt[q]));  // rounded here
+  const float *bias = a.bias + mem * kBias;
+  const uint16_t *W2 = a.w2 + mem * kW2, *W3 = a.w3 + mem * kW2, *W4 = a.w4 + mem * kW4;
+  const uint16_t *W2T = a.w2t + mem * kW2, *W3T = a.w3t + mem * kW2, *W4T = a.w4t + mem * kW4T;
+  const int64_t sH = (int64_t)kTRows * a.Bt, sD = (int64_t)kHid * a.Bt;
+  f32x4 acc[P][C];
+  uint2 s1[P][C], s2[P][C], s3[P][C];
+  float4 b[C];
+  WFrag<C> wf = load_w<C, kInP>(a.w1 + mem * kW1, 0, w, lane);
+  load_bias<C>(bias, w, lq, b);
+  __syncthreads();
+  // inputs, transposed, with the row of ones (kIn) of the bias gradient
+  if (w < Q) {
+    constexpr int KB = Q / 2;
+    const int rb = w / KB, kb = w % KB, f = 16 * rb + lr;
+    const uint16_t *src = xin + (32 * kb + 2 * lq) * kInLd + f;
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = (uint32_t)src[2 * j * kInLd] | (uint32_t)src[(2 * j + 1) * kInLd] << 16;
+      if (f == kIn) v[j] = 0x3f803f80u;
+    }
+    *reinterpret_cast<uint4 *>(a.xt + (int64_t)mem * kInP * a.Bt +
+                               frag(16 * rb, b0 + 32 * kb, a.Bt) + lane * 8) =
+        make_uint4(v[0], v[1], v[2], v[3]);
+  }
+  infer_layer<P, C, 1, kInLd>(xin, a.w1 + mem * kW1, w, lane, wf, acc);
+  wf = load_w<C, kHid>(W2, 0, w, lane);
+  train_epilogue<P, C>(act, acc, b, w, lr, lq, s1);
+  __syncthreads();
+  load_bias<C>(bias + kHid, w, lq, b);
+  infer_layer<P, C, 8, kActLd>(act, W2, w, lane, wf, acc);
+  store_t<Q, 16>(act, kActLd, a.ht[0] + mem * sH, a.Bt, b0, w, lane);
+  wf = load_w<C, kHid>(W3, 0, w, lane);
+  __syncthreads();
+  train_epilogue<P, C>(act, acc, b, w, lr, lq, s2);
+  __syncthreads();
+  load_bias<C>(bias + 2 * kHid, w, lq, b);
+  infer_layer<P, C, 8, kActLd>(act, W3, w, lane, wf, acc);
+  store_t<Q, 16>(act, kActLd, a.ht[1] + mem * sH, a.Bt, b0, w, lane);
+  __syncthreads();
+  train_epilogue<P, C>(act, acc, b, w, lr, lq, s3);
+  wf = load_w<C, kInP>(W4T, 0, w, lane);
+  __syncthreads();
+  // outputs, squared errors (summed in output order) and dL/dY: 16 samples
+  // per wave, outputs 0..3 in lanes 0..15 and 4, 5 in lanes 16..31
+  if (w < Q) {
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      o = mfma(load_w<1, kHid>(W4, kk, 0, lane).v[0],
+               ld8(act + (16 * w + lr) * kActLd + 32 * kk + (lane >> 4) * 8), o);
+    const float4 b4 = *reinterpret_cast<const float4 *>(bias + 3 * kHid + lq);
+    const float r[4] = {o[0] + b4.x - yt[0], o[1] + b4.y - yt[1], o[2] + b4.z - yt[2],
+                        o[3] + b4.w - yt[3]};
+    float e = fmaf(r[0], r[0], r[1] * r[1]);
+    e = fmaf(r[2], r[2], e);
+    e = fmaf(r[3], r[3], e);
+    e = __shfl(e, lr);  // outputs 0..3 of this sample
+    e = fmaf(r[0], r[0], e);
+    e = fmaf(r[1], r[1], e);
+    if (lq == 4) a.loss_v[(int64_t)mem * a.Bt + b0 + 16 * w + lr] = e;
+    if (lq < 8) {
+      const bool six = lq == 0;  // outputs 6 and 7 are padding
+      *reinterpret_cast<uint2 *>(d4 + (16 * w + lr) * kInLd + lq) =
+          pack4(r[0] * a.gscale, r[1] * a.gscale, six ? r[2] * a.gscale : 0.f,
+                six ? r[3] * a.gscale : 0.f);
+    }
+  }
+  store_t<Q, 16>(act, kActLd, a.ht[2] + mem * sH, a.Bt, b0, w, lane);
+  __syncthreads();
+  store_t<Q, 1>(d4, kInLd, a.d4t + (int64_t)mem * kOutP * a.Bt, a.Bt, b0, w, lane);
+  infer_layer<P, C, 1, kInLd>(d4, W4T, w, lane, wf, acc);
+  wf = load_w<C, kHid>(W3T, 0, w, lane);
+  back_epilogue<P, C>(act, acc, w, lr, lq, s3);
+  __syncthreads();
+  infer_layer<P, C, 8, kActLd>(act, W3T, w, lane, wf, acc);
+  store_t<Q, 16>(act, kActLd, a.dt[2] + mem * sD, a.Bt, b0, w, lane);
+  wf = load_w<C, kHid>(W2T, 0, w, lane);
+  __syncthreads();
+  back_epilogue<P, C>(act, acc, w, lr, lq, s2);
+  __syncthreads();
+  infer_layer<P, C, 8, kActLd>(act, W2T, w, lane, wf, acc);
+  store_t<Q, 16>(act, kActLd, a.dt[1] + mem * sD, a.Bt, b0, w, lane);
+  __syncthreads();
+  back_epilogue<P, C>(act, acc, w, lr, lq, s1);
+  __syncthreads();
+  store_t<Q, 16>(act, kActLd, a.dt[0] + mem * sD, a.Bt, b0, w, lane);
+}
+
+// Weight gradients: part_L[split] = D_L^T [H_{L-1}^T; 1] over kSplitK rows of
+// the batch.  Operands in fragment order; a wave takes R blocks of outputs o
+// and N of inputs i and ends with four consecutive i of one o per lane.
+// Bound by memory: 75 MB read and 36 MB written for four members of 4096
+// samples, 24 us (4.6 TB/s); 60 us in 32 x 32 tiles from operands read row by
+// row.  Two k steps in flight instead of four: 26 us.
+struct DwArgs {
+  const uint16_t *xt, *ht[3], *dt[3], *d4t;
+  int Bt;
+  float *part[4];
+};
+constexpr int kSplitK = 256;  // batch rows per K split of the weight gradients
+constexpr int kLdp[4] = {kInP, kTRows, kTRows, kTRows};
+constexpr int kPartM[4] = {kHid, kHid, kHid, kOutP};
+
+template <int R, int N>
+__device__ __forceinline__ void dw_tile(const uint16_t *D, const uint16_t *H, int kb, int ob,
+                                        int ib, float *part, int ld, int lane) {
+  constexpr int KS = kSplitK / 32;
+  f32x4 acc[R][N];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int n = 0; n < N; ++n) acc[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint16_t *pd = D + (int64_t)ob * kb * 512 + lane * 8;
+  const uint16_t *ph = H + (int64_t)ib * kb * 512 + lane * 8;
+  constexpr int DEPTH = 4;  // k steps in flight
+  bf16x8 d[DEPTH][R], h[DEPTH][N];
+#pragma unroll
+  for (int kk = 0; kk < KS + DEPTH - 1; ++kk) {
+    if (kk < KS) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) d[kk % DEPTH][r] = ld8(pd + ((int64_t)r * kb + kk) * 512);
+#pragma unroll
+      for (int n = 0; n < N; ++n) h[kk % DEPTH][n] = ld8(ph + ((int64_t)n * kb + kk) * 512);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int k = kk - (DEPTH - 1);
+    if (k >= 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+          acc[r][n] = mfma(h[k % DEPTH][n], d[k % DEPTH][r], acc[r][n]);
+    }
+  }
+  const int lr = lane & 15, lq = (lane >> 4) * 4;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      *reinterpret_cast<float4 *>(part + (int64_t)(16 * (ob + r) + lr) * ld + 16 * (ib + n) +
+                                  lq) =
+          make_float4(acc[r][n][0], acc[r][n][1], acc[r][n][2], acc[r][n][3]);
+}
+
+// Six units of eight waves per split: two halves of the outputs of layers 2
+// and 3 (waves of 4 x 4 blocks, the last column of waves with the block of
+// ones as a fifth), layer 1 and layer 4.
+constexpr int kDwUnits = 6;
+__global__ __launch_bounds__(512, 2) void dw_kernel(DwArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int unit = blockIdx.x % kDwUnits, split = blockIdx.x / kDwUnits, mem = blockIdx.y;
+  const int kb = a.Bt / 32;
+  const int64_t splits = a.Bt / kSplitK, k0 = (int64_t)split * (kSplitK / 32) * 512, B = a.Bt;
+  if (unit < 4) {
+    const int L = 1 + (unit >> 1);
+    const uint16_t *D = a.dt[L] + mem * kHid * B + k0, *H = a.ht[L - 1] + mem * kTRows * B + k0;
+    float *part = a.part[L] + (mem * splits + split) * (kHid * kTRows);
+    const int ob = 8 * (unit & 1) + 4 * (w >> 2), ib = 4 * (w & 3);
+    if ((w & 3) == 3)
+      dw_tile<4, 5>(D, H, kb, ob, ib, part, kTRows, lane);
+    else
+      dw_tile<4, 4>(D, H, kb, ob, ib, part, kTRows, lane);
+  } else if (unit == 4) {
+    dw_tile<2, 2>(a.dt[0] + mem * kHid * B + k0, a.xt + mem * kInP * B + k0, kb, 2 * w, 0,
+                  a.part[0] + (mem * splits + split) * (kHid * kInP), kInP, lane);
+  } else {
+    const uint16_t *D = a.d4t + mem * kOutP * B + k0, *H = a.ht[2] + mem * kTRows * B + k0;
+    float *part = a.part[3] + (mem * splits + split) * (kOutP * kTRows);
+    if (w == 7)
+      dw_tile<1, 3>(D, H, kb, 0, 14, part, kTRows, lane);
+    else
+      dw_tile<1, 2>(D, H, kb, 0, 2 * w, part, kTRows, lane);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Surrogate path helpers.
 __device__ inline const double *pick_F(const double *F, int nF, int r) {
   return F + 9 * (int64_t)(nF == 1 ? 0 : r);
@@ -678,8 +867,8 @@ struct mf_mlp {
   int64_t adam_t = 0;
   // training workspace for mini-batches of Bt samples
   int Bt = 0;
-  DevBuf<uint16_t> Xn, XnT, H[3], HT[3], S[3], D[3], DT[3], D4, D4T;
-  DevBuf<float> Yt, Yo, part[4], loss_part, loss_out, loss_acc, grad;
+  DevBuf<uint16_t> XT, HT[3], DT[3], D4T;  // operands of the weight gradients
+  DevBuf<float> part[4], loss_v, loss_out, loss_acc, grad;
   DevBuf<int32_t> idx;
   mf_estimator est{};
   double last_ms = 0;
@@ -692,16 +881,12 @@ struct mf_mlp {
 
 namespace {
 
-constexpr int kSplitK = 256;  // batch rows per K split of the weight gradients
-const int kLdp[4] = {kInP, kTRows, kTRows, kTRows};
-const int kPartM[4] = {kHid, kHid, kHid, kOutP};
-
 int upload_norm(mf_mlp *m) {
   MF_HIP(hipMemcpyAsync(m->nm_dev.p, &m->nm, sizeof(MlpNorm), hipMemcpyHostToDevice, m->s));
   return MF_OK;
 }
 
-int run_adam(mf_mlp *m, int mode, float lr, float b1, float b2, float eps) {
+int run_adam(mf_mlp *m, int mode, float lr, float b1, float b2, float eps, bool loss = false) {
   AdamArgs a;
   std::memset(&a, 0, sizeof(a));
   a.P = m->P.p;
@@ -733,7 +918,12 @@ int run_adam(mf_mlp *m, int mode, float lr, float b1, float b2, float eps) {
   }
   a.grad = m->grad.p;
   a.mode = mode;
-  hipLaunchKernelGGL(adam_kernel, dim3((kNumParams + 255) / 256, m->K), dim3(256), 0, m->s,
+  a.loss_v = m->loss_v.p;
+  a.Bt = m->Bt;
+  a.loss_inv = m->Bt > 0 ? 1.0f / (6.0f * (float)m->Bt) : 0.f;
+  a.loss_out = m->loss_out.p;
+  a.loss_acc = m->loss_acc.p;
+  hipLaunchKernelGGL(adam_kernel, dim3(kAdamBlocks + (loss ? 1 : 0), m->K), dim3(256), 0, m->s,
                      a);
   MF_HIP(hipGetLastError());
   return MF_OK;
@@ -743,150 +933,80 @@ int ensure_workspace(mf_mlp *m, int Bt) {
   if (Bt == m->Bt) return MF_OK;
   m->Bt = 0;
   const size_t K = m->K, B = Bt;
-  MF_HIP(m->Xn.alloc(K * B * kInP));
-  MF_HIP(m->XnT.alloc(K * kInP * B));
+  MF_HIP(m->XT.alloc(K * kInP * B));
   for (int l = 0; l < 3; ++l) {
-    MF_HIP(m->H[l].alloc(K * B * kHid));
     MF_HIP(m->HT[l].alloc(K * kTRows * B));
-    MF_HIP(m->S[l].alloc(K * B * kHid));
-    MF_HIP(m->D[l].alloc(K * B * kHid));
     MF_HIP(m->DT[l].alloc(K * kHid * B));
   }
-  MF_HIP(m->D4.alloc(K * B * kInP));
   MF_HIP(m->D4T.alloc(K * kOutP * B));
-  MF_HIP(m->Yt.alloc(K * B * 8));
-  MF_HIP(m->Yo.alloc(K * B * kOutP));
   const size_t splits = B / kSplitK;
   for (int L = 0; L < 4; ++L) MF_HIP(m->part[L].alloc(K * splits * kPartM[L] * kLdp[L]));
-  MF_HIP(m->loss_part.alloc(K * ((B + 255) / 256)));
-  // zero padding (columns / rows that are never written) and ones rows
-  MF_HIP(hipMemsetAsync(m->Xn.p, 0, sizeof(uint16_t) * m->Xn.n, m->s));
-  MF_HIP(hipMemsetAsync(m->XnT.p, 0, sizeof(uint16_t) * m->XnT.n, m->s));
-  MF_HIP(hipMemsetAsync(m->D4.p, 0, sizeof(uint16_t) * m->D4.n, m->s));
-  MF_HIP(hipMemsetAsync(m->D4T.p, 0, sizeof(uint16_t) * m->D4T.n, m->s));
+  MF_HIP(m->loss_v.alloc(K * B));
+  // rows 256..271 of the activations, which no tile writes: one row of ones
   for (int l = 0; l < 3; ++l) {
     MF_HIP(hipMemsetAsync(m->HT[l].p, 0, sizeof(uint16_t) * m->HT[l].n, m->s));
     hipLaunchKernelGGL(ones_row_kernel, dim3((Bt + 255) / 256, m->K), dim3(256), 0, m->s,
                        m->HT[l].p, (int64_t)kTRows * Bt, kHid, Bt);
     MF_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(ones_row_kernel, dim3((Bt + 255) / 256, m->K), dim3(256), 0, m->s,
-                     m->XnT.p, (int64_t)kInP * Bt, kIn, Bt);
-  MF_HIP(hipGetLastError());
   m->Bt = Bt;
   return MF_OK;
 }
 
-template <int EPI>
-int gemm(mf_mlp *m, const GemmArgs &g, int splits) {
-  const int tiles = ((g.M + 31) / 32) * ((g.N + 31) / 32);
-  hipLaunchKernelGGL(gemm_nt<EPI>, dim3((tiles + 3) / 4, splits, m->K), dim3(256), 0, m->s, g);
-  MF_HIP(hipGetLastError());
-  return MF_OK;
-}
-
-GemmArgs gargs(const uint16_t *A, int64_t lda, int64_t sA, const uint16_t *B, int64_t ldb,
-               int64_t sB, int M, int N, int kc) {
-  GemmArgs g;
-  std::memset(&g, 0, sizeof(g));
-  g.A = A;
-  g.lda = lda;
-  g.sA = sA;
-  g.B = B;
-  g.ldb = ldb;
-  g.sB = sB;
-  g.M = M;
-  g.N = N;
-  g.kc = kc;
-  return g;
+template <int Q>
+void launch_train(const TrainArgs &a, int K, hipStream_t s) {
+  hipLaunchKernelGGL(train_kernel<Q>, dim3((unsigned)(a.Bt / (16 * Q)), K),
+                     dim3(64 * kInferWaves), train_lds(Q), s, a);
 }
 
 // Forward, loss and backward of one mini-batch for every member; leaves the
-// weight-gradient partials in m->part and the loss partials in m->loss_part.
+// weight-gradient partials in m->part and the squared errors in m->loss_v.
 int forward_backward(mf_mlp *m, const float *X, const float *Y, int64_t n_data,
                      const int32_t *idx, int64_t idx_stride, int Bt) {
   int e = ensure_workspace(m, Bt);
   if (e != MF_OK) return e;
   const int K = m->K;
-  const int64_t B = Bt;
-  hipStream_t s = m->s;
-  hipLaunchKernelGGL(prep_kernel, dim3((Bt + 255) / 256, K), dim3(256), 0, s, X, Y, n_data,
-                     idx, idx_stride, Bt, m->nm_dev.p, m->Xn.p, m->XnT.p, m->Yt.p);
-  MF_HIP(hipGetLastError());
-  // forward
-  const uint16_t *Ain = m->Xn.p;
-  int64_t lda = kInP, sA = B * kInP;
-  const uint16_t *Wl[3] = {m->w1.p, m->w2.p, m->w3.p};
-  const int64_t ldw[3] = {kInP, kHid, kHid}, sW[3] = {kW1, kW2, kW2};
+  TrainArgs a;
+  a.X = X;
+  a.Y = Y;
+  a.n_data = n_data;
+  a.idx = idx;
+  a.idx_stride = idx_stride;
+  a.Bt = Bt;
+  a.gscale = 2.0f / (6.0f * (float)Bt);
+  a.w1 = m->w1.p;
+  a.w2 = m->w2.p;
+  a.w3 = m->w3.p;
+  a.w4 = m->w4.p;
+  a.w2t = m->w2t.p;
+  a.w3t = m->w3t.p;
+  a.w4t = m->w4t.p;
+  a.bias = m->bias.p;
+  a.nm = m->nm_dev.p;
+  a.xt = m->XT.p;
+  a.d4t = m->D4T.p;
+  a.loss_v = m->loss_v.p;
+  DwArgs d;
+  d.xt = a.xt;
+  d.d4t = a.d4t;
+  d.Bt = Bt;
   for (int l = 0; l < 3; ++l) {
-    GemmArgs g = gargs(Ain, lda, sA, Wl[l], ldw[l], sW[l], Bt, kHid, (int)ldw[l]);
-    g.bias = m->bias.p + l * kHid;
-    g.sbias = kBias;
-    g.O = m->H[l].p;
-    g.OS = m->S[l].p;
-    g.OT = m->HT[l].p;
-    g.ldo = kHid;
-    g.sO = B * kHid;
-    g.ldt = B;
-    g.sOT = kTRows * B;
-    if ((e = gemm<kFwdHidden>(m, g, 1)) != MF_OK) return e;
-    Ain = m->H[l].p;
-    lda = kHid;
-    sA = B * kHid;
+    d.ht[l] = a.ht[l] = m->HT[l].p;
+    d.dt[l] = a.dt[l] = m->DT[l].p;
   }
-  {
-    GemmArgs g = gargs(m->H[2].p, kHid, B * kHid, m->w4.p, kHid, kW4, Bt, kOutP, kHid);
-    g.bias = m->bias.p + 3 * kHid;
-    g.sbias = kBias;
-    g.Y = m->Yo.p;
-    g.ldy = kOutP;
-    g.sY = B * kOutP;
-    if ((e = gemm<kFwdOut>(m, g, 1)) != MF_OK) return e;
-  }
-  const int nblk = (Bt + 255) / 256;
-  hipLaunchKernelGGL(loss_kernel, dim3(nblk, K), dim3(256), 0, s, m->Yo.p, m->Yt.p, Bt,
-                     2.0f / (6.0f * (float)Bt), m->D4.p, m->D4T.p, m->loss_part.p, nblk);
+  for (int L = 0; L < 4; ++L) d.part[L] = m->part[L].p;
+  // 64 samples per workgroup once that fills the chip
+  if ((int64_t)Bt * K >= 64 * kCus)
+    launch_train<4>(a, K, m->s);
+  else
+    launch_train<2>(a, K, m->s);
   MF_HIP(hipGetLastError());
-  // backward through the hidden layers: D_l = (D_{l+1} W_{l+1}) * silu'(Z_l)
-  {
-    const uint16_t *Ad = m->D4.p;
-    int64_t ldd = kInP, sD = B * kInP;
-    const uint16_t *Wt[3] = {m->w4t.p, m->w3t.p, m->w2t.p};
-    const int64_t ldwt[3] = {kInP, kHid, kHid}, sWt[3] = {kW4T, kW2, kW2};
-    for (int t = 0; t < 3; ++t) {
-      const int l = 2 - t;  // hidden layer receiving the gradient
-      GemmArgs g = gargs(Ad, ldd, sD, Wt[t], ldwt[t], sWt[t], Bt, kHid, (int)ldwt[t]);
-      g.Sin = m->S[l].p;
-      g.O = m->D[l].p;
-      g.OT = m->DT[l].p;
-      g.ldo = kHid;
-      g.sO = B * kHid;
-      g.ldt = B;
-      g.sOT = kHid * B;
-      if ((e = gemm<kBwdHidden>(m, g, 1)) != MF_OK) return e;
-      Ad = m->D[l].p;
-      ldd = kHid;
-      sD = B * kHid;
-    }
-  }
-  // weight gradients (+ bias column): part_L = D_L^T [H_{L-1}^T; 1]
-  const int splits = Bt / kSplitK;
-  const uint16_t *Ag[4] = {m->DT[0].p, m->DT[1].p, m->DT[2].p, m->D4T.p};
-  const int64_t sAg[4] = {kHid * B, kHid * B, kHid * B, kOutP * B};
-  const uint16_t *Bg[4] = {m->XnT.p, m->HT[0].p, m->HT[1].p, m->HT[2].p};
-  const int64_t sBg[4] = {kInP * B, kTRows * B, kTRows * B, kTRows * B};
-  for (int L = 0; L < 4; ++L) {
-    GemmArgs g = gargs(Ag[L], B, sAg[L], Bg[L], B, sBg[L], kPartM[L], kLdp[L], kSplitK);
-    g.Y = m->part[L].p;
-    g.ldy = kLdp[L];
-    g.sYsplit = (int64_t)kPartM[L] * kLdp[L];
-    g.sY = g.sYsplit * splits;
-    if ((e = gemm<kPartial>(m, g, splits)) != MF_OK) return e;
-  }
+  hipLaunchKernelGGL(dw_kernel, dim3((unsigned)(Bt / kSplitK * kDwUnits), K), dim3(512), 0, m->s,
+                     d);
+  MF_HIP(hipGetLastError());
   return MF_OK;
 }
 
-constexpr int kCus = 256;  // compute units of the chip
 template <int Q, int NT, int G>
 void launch_infer(const InferArgs &a, hipStream_t s) {
   hipLaunchKernelGGL((infer_kernel<Q, NT, G>),
@@ -1177,12 +1297,8 @@ int mf_mlp_train_step_device(mf_mlp *m, const float *X_dev, const float *Y_dev,
   int e = forward_backward(m, X_dev, Y_dev, n_data, idx_dev, batch, batch);
   if (e != MF_OK) return e;
   m->adam_t += 1;
-  if ((e = run_adam(m, 0, lr, 0.9f, 0.999f, 1e-8f)) != MF_OK) return e;
+  if ((e = run_adam(m, 0, lr, 0.9f, 0.999f, 1e-8f, loss != nullptr)) != MF_OK) return e;
   if (loss) {
-    const int nblk = (batch + 255) / 256;
-    hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(m->K), 0, m->s, m->loss_part.p, nblk,
-                       1.0f / (6.0f * (float)batch), m->loss_out.p, m->loss_acc.p);
-    MF_HIP(hipGetLastError());
     std::vector<float> l(m->K);
     MF_HIP(hipMemcpyAsync(l.data(), m->loss_out.p, sizeof(float) * m->K,
                           hipMemcpyDeviceToHost, m->s));
@@ -1206,7 +1322,6 @@ int mf_mlp_fit_device(mf_mlp *m, const float *X_dev, const float *Y_dev, int64_t
   const int64_t total = steps * tp->epochs;
   std::vector<int32_t> perm((size_t)K * n);
   MF_HIP(m->idx.ensure(perm.size()));
-  const int nblk = (Bt + 255) / 256;
   int64_t it = 0;
   for (int ep = 0; ep < tp->epochs; ++ep) {
     MF_HIP(hipStreamSynchronize(m->s));  // previous epoch done with idx
@@ -1229,10 +1344,7 @@ int mf_mlp_fit_device(mf_mlp *m, const float *X_dev, const float *Y_dev, int64_t
       int e = forward_backward(m, X_dev, Y_dev, n, m->idx.p + st * Bt, n, Bt);
       if (e != MF_OK) return e;
       m->adam_t += 1;
-      if ((e = run_adam(m, 0, lr, tp->beta1, tp->beta2, tp->eps)) != MF_OK) return e;
-      hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(K), 0, m->s, m->loss_part.p, nblk,
-                         1.0f / (6.0f * (float)Bt), m->loss_out.p, m->loss_acc.p);
-      MF_HIP(hipGetLastError());
+      if ((e = run_adam(m, 0, lr, tp->beta1, tp->beta2, tp->eps, true)) != MF_OK) return e;
     }
     if (epoch_loss) {
       std::vector<float> l(K);
@@ -1256,11 +1368,7 @@ int mf_mlp_gradient_device(mf_mlp *m, int32_t member, const float *X_dev, const 
   }
   int e = forward_backward(m, X_dev, Y_dev, n, nullptr, 0, n);
   if (e != MF_OK) return e;
-  if ((e = run_adam(m, 1, 0, 0, 0, 0)) != MF_OK) return e;
-  const int nblk = (n + 255) / 256;
-  hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(m->K), 0, m->s, m->loss_part.p, nblk,
-                     1.0f / (6.0f * (float)n), m->loss_out.p, m->loss_acc.p);
-  MF_HIP(hipGetLastError());
+  if ((e = run_adam(m, 1, 0, 0, 0, 0, true)) != MF_OK) return e;
   MF_HIP(hipMemcpyAsync(grad_host, m->grad.p + (size_t)member * kNumParams,
                         sizeof(float) * kNumParams, hipMemcpyDeviceToHost, m->s));
   float l = 0;

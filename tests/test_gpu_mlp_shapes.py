@@ -1,11 +1,16 @@
 """Surrogate inference cuts small calls finer than large ones (two members at
 a time, two of the six tangent planes per workgroup).  A row's result does not
 depend on the call it is in, so every size gives the rows of one large call bit
-for bit; the large call is checked against the oracle in test_gpu_mlp.py."""
+for bit; the large call is checked against the oracle in test_gpu_mlp.py.
+
+Training takes 64 or 32 samples per workgroup, by the samples of all members
+together: the gradient of a member is the same bits either way, and the
+oracle's within the tolerances that test_gpu_mlp.py derives."""
 import numpy as np
 import pytest
 
 import mumfim_amd as m
+from oracle import mlp_oracle as mo
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +47,28 @@ def test_one_member_of_an_ensemble_small_and_large(ensemble):
         Y, _, J = mlp.predict(X[:100], jacobian=True, member=k)
         np.testing.assert_array_equal(Y, Y0[:100])
         np.testing.assert_array_equal(J, J0[:100])
+
+
+@pytest.mark.parametrize("batch", [256, 4096, 4352, 16384])
+def test_gradient_of_wide_and_narrow_tiles(batch):
+    rng = np.random.default_rng(batch)
+    norm = (rng.normal(0, 0.1, 10).astype(np.float32), rng.uniform(0.5, 2, 10).astype(np.float32),
+            rng.normal(0, 0.1, 6).astype(np.float32), rng.uniform(0.5, 2, 6).astype(np.float32))
+    X = rng.normal(0, 1, (batch, 10)).astype(np.float32)
+    Y = rng.normal(0, 1, (batch, 6)).astype(np.float32)
+    Xd, Yd = m.DeviceArray.from_host(X), m.DeviceArray.from_host(Y)
+    got = []
+    for members in (4, 1):  # member 0 of both starts from the same weights
+        mlp = m.SurrogateMLP(members, 7)
+        mlp.set_normalization(*norm)
+        got.append(mlp.gradient(0, Xd, Yd, batch))
+        P = mlp.get_weights(0)
+    assert got[0][0] == got[1][0]
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    loss, g = got[0]
+    lo, go = mo.loss_and_grad(P, mo.Norm(*norm), X, Y, emulate=True)
+    assert abs(loss - lo) <= 1e-4 * lo
+    ends = [mo.OFF_W1, mo.OFF_B1, mo.OFF_W2, mo.OFF_B2, mo.OFF_W3, mo.OFF_B3, mo.OFF_W4,
+            mo.OFF_B4, mo.NUM_PARAMS]
+    for a, b in zip(ends, ends[1:]):
+        assert np.linalg.norm(g[a:b] - go[a:b]) <= 2e-3 * np.linalg.norm(go[a:b])
