@@ -632,9 +632,11 @@ int64_t group_gstride(const Variant &v, int N) {
 // mode, FP32c register kernels): with S workgroups resident on the device,
 // n solves of equal length take ceil(n / S) rounds, the last partly empty;
 // c chunks per solve take ceil(n c / S) rounds of 1/c the length.  The
-// count minimising that (plus 1% per extra chunk for the state round trip)
-// is chosen, and only when n >= 2 S, so a chunk's predecessor has finished
-// long before it starts.  params.chunks > 0 forces the count, else the
+// count minimising that is chosen, and only when n >= 2 S, so a chunk's
+// predecessor has finished long before it starts.  Each extra chunk costs its
+// solve a start and a state round trip, the time of 60-100 steps (4096 solves
+// of 500 nodes, 100 steps: 0.89, 1.40, 1.97, 2.65 ms in 1 to 4 chunks), and at
+// least 1%: three chunks give 6% at 3000 steps and take 36% at 300.  params.chunks > 0 forces the count, else the
 // autotuner's measured count when it set one.
 int plan_chunks(const mf_batch *b, const Variant &v, size_t lds, int n) {
   if (b->p.mode != MF_MODE_RAMP || v.prec != MF_PREC_FP32C || !(v.flags & kEllInRegs) ||
@@ -649,10 +651,12 @@ int plan_chunks(const mf_batch *b, const Variant &v, size_t lds, int n) {
     return 1;
   const long S = (long)occ * cus;
   if (n < 2 * S) return 1;
+  constexpr double kChunkSteps = 80.0;
   int best = 1;
   double best_t = 1e300;
   for (int c = 1; c <= 4 && c <= b->p.n_steps; ++c) {
-    const double t = (double)((n * (long)c + S - 1) / S) / c * (1.0 + 0.01 * (c - 1));
+    const double extra = std::max(0.01, kChunkSteps / b->p.n_steps);
+    const double t = (double)((n * (long)c + S - 1) / S) / c * (1.0 + extra * (c - 1));
     if (t < best_t - 1e-12) {
       best_t = t;
       best = c;
