@@ -136,8 +136,6 @@ struct RveDev {
   int32_t react_off;
   int32_t n_react;
   int32_t m_free;     // fibers with a free end (the fiber-stream prefix)
-  int32_t n_nl;       // nonlinear ones among them, first, where both laws occur
-  int32_t t_records;
   double c_sound, scale;
   // Reference coordinates in fixed point for the FP32 kernel: X_q =
   // rint(X * xq_scale) fits int32; xq_scale is a power of two.
@@ -146,6 +144,8 @@ struct RveDev {
   // Free nodes of degree above the per-lane fiber count of the
   // register-resident kernel; they are the first n_split free ranks.
   int32_t n_split;
+  int32_t n_nl;       // nonlinear ones among them, first, where both laws occur
+  int32_t t_records;
 };
 
 // Reaction constants as the kernels consume them.

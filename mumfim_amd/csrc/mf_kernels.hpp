@@ -21,16 +21,12 @@ struct SolveArgs {
   const int32_t *slice_base, *slice_D;
   const int32_t *ell_w;
   const double *ell_l0;     // FP64 kernels
-  const double *ell_r0;     // 1 / ell_l0
-  const uint32_t *fs_ab;    // fiber stream: ranks and reaction in one word
-  const double2 *fs_lr;     // fiber stream: l0, 1 / l0
   const float *ell_il;      // FP32 kernels: 1/l0
   const int32_t *fib;       // 2 per fiber (kernel ranks)
   const int32_t *fstream;   // 4 per fiber: ranks a, b and their ELL entries
   const int32_t *ell_fref;  // per ELL entry: fiber record index | sign bit
   const float *fparam;      // 4 per fiber: reference vector, law coefficient
   const ReactDev *reacts;
-  const Law64 *laws;        // FP64 laws of the same reactions
   const double *x_in, *u_in;
   double *x_out, *u_out;
   const double *V;          // per RVE
@@ -71,6 +67,11 @@ struct SolveArgs {
   // (9 per solve) and the stress derivative along it (6 per solve)
   const double *solve_G;
   double *dsigma;
+  // FP64 kernels
+  const double *ell_r0;     // 1 / ell_l0
+  const uint32_t *fs_ab;    // fiber stream: ranks and reaction in one word
+  const double2 *fs_lr;     // fiber stream: l0, 1 / l0
+  const Law64 *laws;        // the laws of reacts
 };
 
 // Floats of chunk state per solve of a register-kernel workgroup of B
