@@ -370,11 +370,12 @@ TuneKey tune_key(int prec, const PackedRVE &p, bool lin) {
                  (p.Nf + p.n_split + 63) / 64, (p.N + 255) / 256};
 }
 
-// Solves of one launch if they are few enough to be all on the chip at once
-// (else 0): up to four per CU.  Then the time is that of one solve's steps, not
-// of the work in all, and a node per thread of a wider workgroup beats more
-// nodes per lane; the sums of a node, hence the results, are the same.  Ramp
-// mode, FP32c (the register kernels); us of 300 steps, narrow against wide:
+// How wide the workgroups of an FP32c ramp launch may be taken for lack of
+// solves to fill the chip: threads per solve with one node each, 0 for the
+// ranking below.  With every solve on the chip at once the time is that of one
+// solve's steps, not of the work in all, and a node per thread beats several
+// per lane; a node's sums, hence the results, are the same.  us of 300 steps,
+// narrow against wide:
 //   at most one solve per CU, 512 threads (768 with toe-law fibers, where the
 //   table lookups want registers): 180 nodes 423 -> 203 (toe 798 -> 347),
 //   250 nodes 298 -> 209 (445 -> 360), 400 nodes 322 -> 219 (401 -> 368);
@@ -384,8 +385,10 @@ TuneKey tune_key(int prec, const PackedRVE &p, bool lin) {
 //   at most four, 256 threads instead of one RVE per wave, 1024 solves: 120
 //   nodes 417 -> 257 (766 -> 456), 180 nodes 455 -> 293 (888 -> 513); 1536
 //   solves: 476 -> 474, and slower from there.
+// The last two only where every RVE of the batch fits: beside larger RVEs the
+// wider workgroups take their room (700 solves of 200 to 500 nodes: 542 -> 594).
 constexpr int kCus = 256;  // compute units of the chip
-long few_solves(const mf_batch *b, int prec) {
+int wide_threads(const mf_batch *b, int prec) {
   if (prec != MF_PREC_FP32C || b->p.mode != MF_MODE_RAMP) return 0;
   // FP32c differences put all perturbed solves of a tangent in one launch
   const long per = b->p.tangent_precision != MF_PREC_FP32C ||
@@ -393,7 +396,11 @@ long few_solves(const mf_batch *b, int prec) {
                        ? 1
                    : b->p.tangent_scheme == MF_TANGENT_CENTRAL ? 13
                                                                : 7;
-  return b->R * per <= 4L * kCus ? b->R * per : 0;
+  const long n = b->R * per;
+  if (n <= kCus) return 768;
+  int lanes = 0;
+  for (const PackedRVE &p : b->host) lanes = std::max(lanes, p.Nf + p.n_split);
+  return n <= 2 * kCus && lanes <= 448 ? 512 : n <= 4 * kCus && lanes <= 256 ? 256 : 0;
 }
 
 // Picks the kernel variant of every RVE for one precision: the autotuned
@@ -405,7 +412,7 @@ int make_plan(mf_batch *b, int prec) {
   const Variant *vs = variants(&nv);
   b->plan[prec].assign(b->R, -1);
   b->lds[prec].assign(b->R, 0);
-  const long few = few_solves(b, prec);
+  const int wide = wide_threads(b, prec);
   for (int r = 0; r < b->R; ++r) {
     const PackedRVE &p = b->host[r];
     const bool lin = all_linear(p);
@@ -449,10 +456,8 @@ int make_plan(mf_batch *b, int prec) {
       // RVEs (four RVEs per workgroup) and 5% on toe-law ones (one)
       const bool wave = (v.flags & kWaveRve) != 0;
       const long wave_rank = lin ? (v.block == 256 ? 0 : 10) : (v.block == 64 ? 0 : 10);
-      const bool wide = few > 0 && regs && !wave && v.npt == 1 && v.block <= 768 &&
-                        (few <= kCus       ? v.block >= 512
-                         : few <= 2 * kCus ? v.block == 512 && p.Nf + p.n_split <= 448
-                                           : v.block == 256);
+      const bool widen = wide > 0 && regs && !wave && v.npt == 1 &&
+                         (wide == 768 ? v.block >= 512 && v.block <= 768 : v.block == wide);
       // global-state FP64 last: only where nothing else fits.  FP64 with each
       // fiber evaluated once before the node-centric FP64 kernels for RVEs
       // with toe-law fibers (11% on 1500-node RVEs), after them for linear
@@ -467,7 +472,7 @@ int make_plan(mf_batch *b, int prec) {
                  : fpar ? (lin ? 50000000L : 15000000L) + fpl * 100000 + (long)v.block * 10 + mode_rank
                  : fstr ? (lin ? 55000000L : 15350000L) + (v.block > 768 ? 50000L : 0L) +
                               (long)v.npt * 10000 + fpl * 100 + mode_rank
-                 : wide ? 4000000L + 10 * (lin ? v.block : 1024 - v.block) + mode_rank
+                 : widen ? 4000000L + 10 * (lin ? v.block : 1024 - v.block) + mode_rank
                  : wave ? 5000000L + wave_rank + mode_rank
                  : reg256x2 ? 10000000L + 5000
                  : regbig_nl ? 15340000L + mode_rank
