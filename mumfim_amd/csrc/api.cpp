@@ -496,7 +496,14 @@ int make_plan(mf_batch *b, int prec) {
 
 // Tangent-linear variant of every RVE: three directions per workgroup where
 // its LDS holds them, then the fewest node slots per thread, then the fewest
-// threads, that hold its free nodes.
+// threads, that hold its free nodes.  While the six workgroups of every RVE
+// with one direction each find room (one per CU; three of 256 threads), the
+// shared base solve saves nothing and one direction's steps are shorter.  ms of
+// 200 steps, three against one, linear fibers: 42 RVEs of 400 nodes 1.20, 1.07,
+// 750 nodes 1.12, 1.07, 1800 nodes 2.35, 1.51; 43 RVEs of 750 nodes 1.14, 1.55;
+// 128 RVEs of 200 nodes 1.72, 1.61 and 256 of them 2.61, 3.05.  Linear RVEs
+// beyond two nodes per thread, whose three directions leave few registers: 64
+// of 1800 nodes 2.50, 2.44, 85 of them 2.68, 2.76 (toe 64: 2.63, 2.87).
 void make_plan_tl(mf_batch *b) {
   int nv = 0;
   const Variant *vs = variants(&nv);
@@ -504,13 +511,18 @@ void make_plan_tl(mf_batch *b) {
   b->lds_tl.assign(b->R, 0);
   for (int r = 0; r < b->R; ++r) {
     const PackedRVE &p = b->host[r];
+    const long room = p.Nf <= 256                       ? 3 * kCus
+                      : p.Nf > 2 * 768 && all_linear(p) ? 3 * kCus / 2
+                                                        : kCus;
+    const bool spread = 6L * b->R <= room;
     long best_key = 0;
     for (int i = 0; i < nv; ++i) {
       const Variant &v = vs[i];
       if (!(v.flags & kTangentLinear) || (long)v.block * v.npt < p.Nf) continue;
       const size_t L = lds_bytes(v, p.N, p.Nb, p.M, p.ell_free_entries, p.t_records);
       if (L > kMaxLds) continue;
-      const long key = (tl_dirs(v.flags) > 1 ? 0L : 10000000L) + (long)v.npt * 100000 + v.block;
+      const long key = ((tl_dirs(v.flags) > 1) != spread ? 0L : 10000000L) +
+                       (long)v.npt * 100000 + v.block;
       if (b->plan_tl[r] < 0 || key < best_key) {
         b->plan_tl[r] = i;
         b->lds_tl[r] = L;

@@ -66,3 +66,29 @@ def test_tables_and_boundaries(kind):
     else:
         net.boundary = np.arange(net.n_nodes, dtype=np.int32)
     check([net, net])
+
+
+@pytest.mark.parametrize("law", [0.0, 0.5, 1.0])
+@pytest.mark.parametrize("sizes", [[20, 286, 290, 294], [573, 580, 586], [865, 872, 1730, 1742],
+                                   [2150, 2250]])
+def test_few_and_many(sizes, law):
+    """Small batches take one direction per workgroup, large ones three: the
+    same trajectory and derivatives, so stress and tangent agree up to the order
+    of their FP64 sums over the boundary nodes, which follows the thread count."""
+    say(f"case: few and many, sizes {sizes} law {law}")
+    nets = [mf.generate_network(seed=500 + n, n_nodes=n, nonlinear_fraction=law) for n in sizes]
+    p = mf.default_params(mode=mf.MF_MODE_RAMP, n_steps=120, precision=mf.MF_PREC_FP32C,
+                          reaction_policy=mf.MF_REACT_PER_FIBER,
+                          tangent_scheme=mf.MF_TANGENT_LINEAR,
+                          tangent_precision=mf.MF_PREC_FP32C)
+    F = strain(3, len(nets), 0.05)
+    few = mf.BatchedFiberRVEAnalysisExplicit(nets, p)
+    copies = 132 // len(nets)  # more than 128 RVEs: beyond both lines
+    many = mf.BatchedFiberRVEAnalysisExplicit(nets * copies, p)
+    s1, C1 = few.run_with_tangent(F)
+    s3, C3 = many.run_with_tangent(np.tile(F, (copies, 1, 1)))
+    n = len(nets)
+    for k in (0, copies - 1):
+        for many_, few_ in ((C3, C1), (s3, s1)):
+            np.testing.assert_allclose(np.asarray(many_)[k * n:(k + 1) * n], few_, rtol=0,
+                                       atol=1e-13 * np.abs(few_).max())
