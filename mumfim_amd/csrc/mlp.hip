@@ -1008,11 +1008,23 @@ int forward_backward(mf_mlp *m, const float *X, const float *Y, int64_t n_data,
   return MF_OK;
 }
 
+// A grid dimension counts its threads in 32 bits and wraps silently, so calls of
+// more than 2^21 tiles (at most 2^31 threads; 2^25 rows with a Jacobian, 2^27 without)
+// take several launches, each of whole tiles.
 template <int Q, int NT, int G>
-void launch_infer(const InferArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((infer_kernel<Q, NT, G>),
-                     dim3((unsigned)((a.n + 16 * Q - 1) / (16 * Q)), NT ? 6 / NT : 1),
-                     dim3(64 * kInferWaves * G), infer_lds(Q * (1 + NT), G), s, a);
+void launch_infer(InferArgs a, hipStream_t s) {
+  constexpr int64_t kRows = (int64_t)(1 << 21) * 16 * Q;
+  static_assert(64 * kInferWaves * G * (kRows / (16 * Q)) <= (int64_t)UINT32_MAX, "threads");
+  for (int64_t left = a.n; left > 0; left -= kRows) {
+    a.n = std::min(left, kRows);
+    hipLaunchKernelGGL((infer_kernel<Q, NT, G>),
+                       dim3((unsigned)((a.n + 16 * Q - 1) / (16 * Q)), NT ? 6 / NT : 1),
+                       dim3(64 * kInferWaves * G), infer_lds(Q * (1 + NT), G), s, a);
+    a.X += kRows * kIn;
+    a.Y += kRows * kOut;
+    if (a.J) a.J += kRows * 36;
+    if (a.spread) a.spread += kRows * kOut;
+  }
 }
 template <int Q, int NT, int G>
 hipError_t infer_attr() {
