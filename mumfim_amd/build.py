@@ -28,6 +28,7 @@ SOURCES = {
     # constants of the exponential stay where they are used: moved out of the
     # step loop they take some 30 registers a lane, which then spill
     "solve64.hip": ["-ffp-contract=off", "-mllvm", "-disable-machine-licm"],
+    "solve64l.hip": ["-ffp-contract=off"],
     "solve32.hip": [],
     # values stay where they are used: moved out of the step loop they spill
     "solve32t.hip": ["-mllvm", "-disable-machine-licm"],
