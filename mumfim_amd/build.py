@@ -30,8 +30,9 @@ SOURCES = {
     "solve64.hip": ["-ffp-contract=off", "-mllvm", "-disable-machine-licm"],
     "solve64l.hip": ["-ffp-contract=off"],
     "solve32.hip": [],
+    "solve32t.hip": [],
     # values stay where they are used: moved out of the step loop they spill
-    "solve32t.hip": ["-mllvm", "-disable-machine-licm"],
+    "solve32tk.hip": ["-mllvm", "-disable-machine-licm"],
     "mlp.hip": [],
 }
 

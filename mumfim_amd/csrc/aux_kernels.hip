@@ -236,6 +236,7 @@ static const Variant kVariants[] = {
     // FP32c tangent-linear: (threads, free nodes per thread)
 #define MF_TL_ENTRY(B, N) {MF_PREC_FP32C, B, N, kTangentLinear},
     MF_TL_LIST(MF_TL_ENTRY)
+    MF_TL_K_LIST(MF_TL_ENTRY)
 #undef MF_TL_ENTRY
 #define MF_TLK_ENTRY(B, N) {MF_PREC_FP32C, B, N, kTangentLinear | (kTlDirs << kFplShift)},
     MF_TLK_LIST(MF_TLK_ENTRY)

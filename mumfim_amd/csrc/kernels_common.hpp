@@ -423,8 +423,10 @@ struct Lin64 {
 }  // namespace kern
 }  // namespace mf
 
-// Tangent-linear FP32c variants: (threads, free-node slots per thread).
-#define MF_TL_LIST(X) X(256, 1) X(512, 1) X(1024, 1) X(1024, 2) X(1024, 3)
+// Tangent-linear FP32c variants: (threads, free-node slots per thread); the
+// second list is compiled with the variants below (solve32tk.hip).
+#define MF_TL_LIST(X) X(1024, 1) X(1024, 2)
+#define MF_TL_K_LIST(X) X(256, 1) X(512, 1) X(1024, 3)
 
 // The same with kTlDirs directions per workgroup.
 #define MF_TLK_LIST(X) X(256, 1) X(512, 1) X(768, 1) X(768, 2) X(768, 3)
