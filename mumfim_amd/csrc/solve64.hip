@@ -2,38 +2,15 @@
 // compiled with -ffp-contract=off so every product and sum rounds as in the
 // reference C++ (BatchedFiberRVEAnalysisExplicitTeamOuterLoop.h:180-437,
 // BatchedFiberRVEAnalysisExplicitBase.h:155-287).
+#include "root64.hpp"
 #include "solve64_ieee.hpp"
 
 namespace mf {
 namespace kern {
 
-// ---- correctly rounded square roots and quotients, without range handling ---
-// For operands far inside the FP64 range (fast64 RVEs) the scaling and special
-// cases of the compiler's IEEE sequences fall away, and a reciprocal that is
-// at hand replaces the one each division computes.
-//
-// a / b from a reciprocal rb of b that is good to a few units of its last
-// place: the quotient of the first product is within a few ulp, its remainder
-// is formed by an FMA (exact but for a few bits below its own precision) and
-// corrects it.  What is rounded last differs from a / b by at most about
-// 2^-51 ulp, and quotients that close to a rounding boundary are as rare.
-__device__ inline double div64(double a, double b, double rb) {
-  const double q = a * rb;
-  return __builtin_fma(__builtin_fma(-q, b, a), rb, q);
-}
-// l = sqrt(x) and rl = 1 / l to a few units of its last place: Goldschmidt's
-// coupled iteration from the hardware's reciprocal square root, then two
-// Newton corrections of l with an exact remainder.  x = 0 gives NaN (its
-// quotient by l would be one as well).
+// l = sqrt(x) and rl = 1 / l from the hardware's reciprocal square root
 __device__ inline void sqrt64(double x, double &l, double &rl) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = __builtin_fma(-h, g, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  l = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  rl = h + h;
+  root64(x, __builtin_amdgcn_rsq(x), l, rl);
 }
 // Force of a nonlinear fiber (react64 with the stretch lr, g = (lr^2 - 1)/2
 // and 1/l0 at hand): both extensions are one formula with selected constants.
