@@ -466,7 +466,7 @@ int make_plan(mf_batch *b, int prec) {
       long key = (v.flags & kGlobalState) ? 2000000000L
                  : (v.flags & kFast64)
                      ? ((v.flags & kFiberOnce) ? 600000000L : 700000000L) +
-                           (long)v.npt * 10000000 + (long)v.block * 1000
+                           (long)v.npt * 10000000 + (1024L - v.block) * 1000
                  : (v.flags & kFiberOnce)
                      ? 500000000L + (long)v.npt * 10000000 + (long)v.block * 1000 + mode_rank
                  : fpar ? (lin ? 50000000L : 15000000L) + fpl * 100000 + (long)v.block * 10 + mode_rank

@@ -229,7 +229,7 @@ static const Variant kVariants[] = {
     MF_NODE64_LIST(MF_NODE64_ENTRY)
 #undef MF_NODE64_ENTRY
 #define MF_FONCE_L_ENTRY(B, N) {MF_PREC_FP64, B, N, kFiberOnce | kFast64},
-    MF_NODE64_LIST(MF_FONCE_L_ENTRY)
+    MF_TREC64_LIST(MF_FONCE_L_ENTRY)
 #undef MF_FONCE_L_ENTRY
     // FP64 with the state in global memory: RVEs no other variant holds
     {MF_PREC_FP64, 1024, 1, kGlobalState},

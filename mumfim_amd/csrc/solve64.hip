@@ -720,7 +720,7 @@ void solve64n(SolveArgs a) {
 // node-centric kernel below, which evaluates every fiber twice, in waves of
 // mixed laws, and 20.4 ms with solve64.
 template <int B, int NPT>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(B / 256)))
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4)))
 void solve64t(SolveArgs a) {
 #pragma clang fp contract(off)
   constexpr int NW = B / kWave;
@@ -1302,7 +1302,7 @@ hipError_t launch_solve64(const Variant &v, const SolveArgs &a, int n_blocks,
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(B), lds, s, a);               \
     return hipGetLastError();                                                \
   }
-  MF_NODE64_LIST(MF_FONCE_L_LAUNCH)
+  MF_TREC64_LIST(MF_FONCE_L_LAUNCH)
 #undef MF_FONCE_L_LAUNCH
   if (v.block == 1024 && v.flags == kGlobalState) {
     auto k = kern::solve64g<1024>;
