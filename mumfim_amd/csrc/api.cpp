@@ -605,16 +605,10 @@ int upload_batch(mf_batch *b) {
   MF_HIP(b->slice_D.upload(sD, s));
   MF_HIP(b->ell_w.upload(ew, s));
   MF_HIP(b->ell_l0.upload(ell_l0, s));
-  MF_HIP(b->ell_r0.alloc(ell_l0.size()));
-  MF_HIP(launch_reciprocal(b->ell_l0.p, b->ell_r0.p, (int64_t)ell_l0.size(), s));
   MF_HIP(b->ell_il.upload(il, s));
   MF_HIP(b->fib.upload(fib, s));
   MF_HIP(b->fstream.upload(fst, s));
   MF_HIP(b->ell_fref.upload(efr, s));
-  MF_HIP(b->fs_ab.alloc((size_t)fib_off));
-  MF_HIP(b->fs_lr.alloc((size_t)fib_off));
-  MF_HIP(launch_stream64(b->rves.p, R, b->fstream.p, b->ell_w.p, b->ell_l0.p, b->fs_ab.p,
-                         b->fs_lr.p, s));
   MF_HIP(b->fparam.upload(fpm, s));
   MF_HIP(b->reacts.upload(rx, s));
   MF_HIP(b->laws.alloc(rx.size()));
@@ -630,6 +624,25 @@ int upload_batch(mf_batch *b) {
   MF_HIP(b->cur_stress.alloc(6 * (size_t)R));
   MF_HIP(b->lastF_dev.alloc(9 * (size_t)R));
   MF_HIP(hipStreamSynchronize(s));
+  return MF_OK;
+}
+
+// The arrays that only the streaming FP64 kernels read, formed the first time
+// that variant v is to run (with the tables of run() if run() uses it, so that no
+// launch of run() allocates): 20 bytes per fiber with t records, 8 per list entry
+// node-centric, 1.9 GB together for 16384 RVEs of 200 to 4000 nodes.
+int stream64_arrays(mf_batch *b, const Variant &v) {
+  if (!(v.flags & kFast64)) return MF_OK;
+  if ((v.flags & kFiberOnce) && !b->fs_lr.p) {
+    const size_t fibers = b->fstream.n / 4;
+    MF_HIP(b->fs_ab.alloc(fibers));
+    MF_HIP(b->fs_lr.alloc(fibers));
+    MF_HIP(launch_stream64(b->rves.p, b->R, b->fstream.p, b->ell_w.p, b->ell_l0.p, b->fs_ab.p,
+                           b->fs_lr.p, b->stream));
+  } else if (!(v.flags & kFiberOnce) && !b->ell_r0.p) {
+    MF_HIP(b->ell_r0.alloc(b->ell_l0.n));
+    MF_HIP(launch_reciprocal(b->ell_l0.p, b->ell_r0.p, (int64_t)b->ell_l0.n, b->stream));
+  }
   return MF_OK;
 }
 
@@ -840,6 +853,13 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
   const int nu = (int)order.size();  // workgroups
   MF_HIP(hipMemcpyAsync(b->order.p, order.data(), sizeof(int32_t) * nu,
                         hipMemcpyHostToDevice, s));
+  int nv = 0;
+  const Variant *vs = variants(&nv);
+  for (int i = 0; i < nu; ++i)
+    if (i == 0 || plan[S.rve[order[i]]] != plan[S.rve[order[i - 1]]]) {
+      const int e = stream64_arrays(b, vs[plan[S.rve[order[i]]]]);
+      if (e != MF_OK) return e;
+    }
   SolveArgs a;
   std::memset(&a, 0, sizeof(a));
   a.rves = b->rves.p;
@@ -888,8 +908,6 @@ int launch_set(mf_batch *b, const SolveSet &S, const double *x_in,
   std::vector<std::pair<int, int>> groups;
   std::vector<size_t> glds;
   std::vector<int64_t> ggs;
-  int nv = 0;
-  const Variant *vs = variants(&nv);
   for (int i = 0; i < nu;) {
     int v = plan[S.rve[order[i]]];
     int j = i;
@@ -975,6 +993,10 @@ int build_identity_tables(mf_batch *b) {
         ++j;
       }
       b->id_groups[prec].push_back({v, j - i});
+      if (prec == b->p.precision) {
+        const int e = stream64_arrays(b, vs[v]);
+        if (e != MF_OK) return e;
+      }
       b->id_group_lds[prec].push_back(L);
       b->id_group_gs[prec].push_back(group_gstride(vs[v], maxN));
       gtotal += (size_t)(j - i) * (size_t)b->id_group_gs[prec].back();
