@@ -1607,12 +1607,13 @@ int mf_batch_set_params(mf_batch *b, const mf_solver_params *params) {
   const int old_bs = b->p.block_size;
   const int old_en = b->p.energy_diagnostics;
   const int old_fk = b->p.fp32_kernel;
+  const int old_wide = wide_threads(b, MF_PREC_FP32C);
   b->p = *params;
   if (mode_changed) {
     b->have_prev = false;
   }
   if (old_bs != params->block_size || old_en != params->energy_diagnostics ||
-      old_fk != params->fp32_kernel)
+      old_fk != params->fp32_kernel || old_wide != wide_threads(b, MF_PREC_FP32C))
     for (int prec = 0; prec < 2; ++prec) {
       int e = make_plan(b, prec);
       if (e != MF_OK) return e;
