@@ -290,6 +290,10 @@ int mf_batch_rve_sizes(const mf_batch *b, int32_t *sizes);
  * (params.chunks).
  * Returns the number of distinct launch groups. */
 int mf_batch_plan(mf_batch *b, int32_t *plan);
+/* The tangent-linear kernel of each RVE (MF_TANGENT_LINEAR), 4 ints per RVE:
+ * threads, free-node slots per thread, directions per workgroup (1 or 3), LDS
+ * bytes; threads 0 where none holds the RVE. */
+int mf_batch_tangent_plan(mf_batch *b, int32_t *plan);
 
 /* ---- device memory (no reference counterpart) ----------------------------- */
 /* Plain HBM buffers for the *_device entry points, allocated by the same HIP

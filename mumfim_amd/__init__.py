@@ -117,6 +117,7 @@ SIGNATURES = {
     "mf_batch_get_state": (C.c_int, [_P, _D, _D, _D]),
     "mf_batch_set_state": (C.c_int, [_P, _D, _D, _D]),
     "mf_batch_plan": (C.c_int, [_P, _IP]),
+    "mf_batch_tangent_plan": (C.c_int, [_P, _IP]),
     "mf_batch_rve_sizes": (C.c_int, [_P, _IP]),
     "mf_default_gen_params": (None, [C.POINTER(mf_gen_params)]),
     "mf_generate_network": (C.c_int, [C.POINTER(mf_gen_params), _IP, _IP, _IP, _D, _IP, _IP, _IP, C.POINTER(mf_reaction)]),
@@ -510,6 +511,12 @@ class BatchedFiberRVEAnalysisExplicit:
         p = np.zeros((self.n, 4), np.int32)
         ng = lib().mf_batch_plan(self.h, _iptr(p))
         return ng, p
+
+    def tangent_plan(self):
+        """Tangent-linear kernel per RVE: threads, node slots, directions, LDS bytes."""
+        p = np.zeros((self.n, 4), np.int32)
+        check(lib().mf_batch_tangent_plan(self.h, _iptr(p)))
+        return p
 
 
 def _fptr(a):

@@ -2250,6 +2250,20 @@ int mf_batch_plan(mf_batch *b, int32_t *plan) {
   return (int)seen.size();
 }
 
+int mf_batch_tangent_plan(mf_batch *b, int32_t *plan) {
+  if (!b || !plan) return MF_ERR_INVALID;
+  int nv = 0;
+  const Variant *vs = variants(&nv);
+  for (int r = 0; r < b->R; ++r) {
+    const int v = b->plan_tl[r];
+    plan[4 * r + 0] = v < 0 ? 0 : vs[v].block;
+    plan[4 * r + 1] = v < 0 ? 0 : vs[v].npt;
+    plan[4 * r + 2] = v < 0 ? 0 : tl_dirs(vs[v].flags);
+    plan[4 * r + 3] = v < 0 ? 0 : (int32_t)b->lds_tl[r];
+  }
+  return MF_OK;
+}
+
 int mf_generate_network(const mf_gen_params *g, int32_t *n_nodes,
                         int32_t *n_fibers, int32_t *n_boundary, double *coords,
                         int32_t *fibers, int32_t *fiber_reaction,
