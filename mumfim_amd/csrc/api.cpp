@@ -252,6 +252,7 @@ struct mf_batch {
   DevBuf<double> gstate;  // global-state variants' per-solve scratch
   size_t id_gtotal[2] = {0, 0};  // doubles of global state of a one-solve-per-RVE run
   int device = 0;                // HIP device the batch lives on
+  int cus = device_cus();        // its compute units
   DevBuf<double> lastF_dev;
   bool lastF_on_device = false;
   // energies of the last run() (FP64 energy diagnostics), 4 per RVE
@@ -387,7 +388,6 @@ TuneKey tune_key(int prec, const PackedRVE &p, bool lin) {
 //   solves: 476 -> 474, and slower from there.
 // The last two only where every RVE of the batch fits: beside larger RVEs the
 // wider workgroups take their room (700 solves of 200 to 500 nodes: 542 -> 594).
-constexpr int kCus = 256;  // compute units of the chip
 int wide_threads(const mf_batch *b, int prec) {
   if (prec != MF_PREC_FP32C || b->p.mode != MF_MODE_RAMP) return 0;
   // FP32c differences put all perturbed solves of a tangent in one launch
@@ -397,10 +397,11 @@ int wide_threads(const mf_batch *b, int prec) {
                    : b->p.tangent_scheme == MF_TANGENT_CENTRAL ? 13
                                                                : 7;
   const long n = b->R * per;
-  if (n <= kCus) return 768;
+  const long cus = b->cus;
+  if (n <= cus) return 768;
   int lanes = 0;
   for (const PackedRVE &p : b->host) lanes = std::max(lanes, p.Nf + p.n_split);
-  return n <= 2 * kCus && lanes <= 448 ? 512 : n <= 4 * kCus && lanes <= 256 ? 256 : 0;
+  return n <= 2 * cus && lanes <= 448 ? 512 : n <= 4 * cus && lanes <= 256 ? 256 : 0;
 }
 
 // Picks the kernel variant of every RVE for one precision: the autotuned
@@ -511,9 +512,9 @@ void make_plan_tl(mf_batch *b) {
   b->lds_tl.assign(b->R, 0);
   for (int r = 0; r < b->R; ++r) {
     const PackedRVE &p = b->host[r];
-    const long room = p.Nf <= 256                       ? 3 * kCus
-                      : p.Nf > 2 * 768 && all_linear(p) ? 3 * kCus / 2
-                                                        : kCus;
+    const long room = p.Nf <= 256                       ? 3L * b->cus
+                      : p.Nf > 2 * 768 && all_linear(p) ? 3L * b->cus / 2
+                                                        : b->cus;
     const bool spread = 6L * b->R <= room;
     long best_key = 0;
     for (int i = 0; i < nv; ++i) {
@@ -675,11 +676,8 @@ int plan_chunks(const mf_batch *b, const Variant &v, size_t lds, int n) {
   const int force = b->p.chunks > 0 ? b->p.chunks : b->tuned_chunks;
   if (force > 0) return std::max(1, std::min(force, b->p.n_steps));
   const int occ = chunk_occupancy(v, lds);
-  int cus = 0;
-  if (occ <= 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) !=
-                      hipSuccess || cus <= 0)
-    return 1;
-  const long S = (long)occ * cus;
+  if (occ <= 0) return 1;
+  const long S = (long)occ * b->cus;
   if (n < 2 * S) return 1;
   constexpr double kChunkSteps = 80.0;
   int best = 1;

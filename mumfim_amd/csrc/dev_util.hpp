@@ -19,6 +19,16 @@
 
 namespace mf {
 
+// Compute units of the current device (256 on an MI355X in one partition); that
+// number too where none can be asked.
+inline int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+    return n;
+  return 256;
+}
+
 template <class T>
 struct DevBuf {
   T *p = nullptr;

@@ -55,7 +55,6 @@ __host__ __device__ constexpr int64_t frag(int64_t row, int64_t k, int64_t kp) {
   return ((row >> 4) * (kp >> 5) + (k >> 5)) * 512 + (((k & 31) >> 3) * 16 + (row & 15)) * 8 +
          (k & 7);
 }
-constexpr int kCus = 256;           // compute units of the chip
 constexpr int kActLd = kHid + 8;  // LDS row stride (BF16) of the inference tile
 
 __device__ __forceinline__ uint16_t bf(float x) {
@@ -858,6 +857,7 @@ using namespace mf::mlpk;
 
 struct mf_mlp {
   int K = 1;
+  int cus = device_cus();  // compute units of the device it lives on
   hipStream_t s = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   DevBuf<float> P, Mo, Ve, bias;
@@ -997,7 +997,7 @@ int forward_backward(mf_mlp *m, const float *X, const float *Y, int64_t n_data,
   }
   for (int L = 0; L < 4; ++L) d.part[L] = m->part[L].p;
   // 64 samples per workgroup once that fills the chip
-  if ((int64_t)Bt * K >= 64 * kCus)
+  if ((int64_t)Bt * K >= 64 * m->cus)
     launch_train<4>(a, K, m->s);
   else
     launch_train<2>(a, K, m->s);
@@ -1094,11 +1094,11 @@ int mlp_predict(mf_mlp *m, int member, const float *X, int64_t n, float *Y, floa
   // 42 -> 29.5 us (5600 points: 42 against 42).
   const int64_t t16 = (n + 15) / 16;
   if (J) {
-    if (3 * t16 <= kCus)
+    if (3 * t16 <= m->cus)
       launch_infer<1, 2, 2>(a, s);
     else
       launch_infer<1, 6, 1>(a, s);
-  } else if (t16 <= kCus) {
+  } else if (t16 <= m->cus) {
     launch_infer<1, 0, 2>(a, s);
   } else {
     launch_infer<4, 0, 1>(a, s);
