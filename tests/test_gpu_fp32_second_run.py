@@ -50,3 +50,22 @@ def test_second_run(n, law, kw, shape, mode):
     err = [float(np.abs(a - b).max()) for a, b in zip(x32, x64)]
     print(f"  error of the positions: first {err[0]:.2e}, second {err[1]:.2e}", flush=True)
     assert err[0] <= 1e-6 and err[1] <= 1e-6
+
+
+@pytest.mark.parametrize("n,law", [(130, 0.5), (180, 0.0), (250, 0.0), (400, 1.0)])
+def test_second_run_does_not_depend_on_the_size_of_its_batch(n, law):
+    """Small batches run a node per lane, large ones several: the same bits."""
+    print(f"case: {n} nodes law {law}", flush=True)
+    net = mf.generate_network(seed=77, n_nodes=n, nonlinear_fraction=law)
+    p = mf.default_params(mode=mf.MF_MODE_RAMP, n_steps=60, precision=mf.MF_PREC_FP32C,
+                          reaction_policy=mf.MF_REACT_PER_FIBER)
+    got = []
+    for R in (1, 1100):
+        g = mf.BatchedFiberRVEAnalysisExplicit([net] * R, p)
+        for seed in (5, 6):
+            u = np.random.default_rng(seed).uniform(-0.08, 0.08, (1, 3, 3))
+            g.run(np.repeat(np.eye(3)[None] + 0.5 * (u + u.transpose(0, 2, 1)), R, 0))
+        got.append((g.plan()[1][0, :3].tolist(), g.get_state()[0][:n]))
+        g.close()
+    assert got[0][0] != got[1][0]  # different kernels
+    np.testing.assert_array_equal(got[0][1], got[1][1])
