@@ -500,21 +500,31 @@ int make_plan(mf_batch *b, int prec) {
 // threads, that hold its free nodes.  While the six workgroups of every RVE
 // with one direction each find room (one per CU; three of 256 threads), the
 // shared base solve saves nothing and one direction's steps are shorter.  ms of
-// 200 steps, three against one, linear fibers: 42 RVEs of 400 nodes 1.20, 1.07,
-// 750 nodes 1.12, 1.07, 1800 nodes 2.35, 1.51; 43 RVEs of 750 nodes 1.14, 1.55;
-// 128 RVEs of 200 nodes 1.72, 1.61 and 256 of them 2.61, 3.05.  Linear RVEs
-// beyond two nodes per thread, whose three directions leave few registers: 64
-// of 1800 nodes 2.50, 2.44, 85 of them 2.68, 2.76 (toe 64: 2.63, 2.87).
+// 200 steps, three against one, linear fibers: 42 RVEs of 400 nodes 1.20, 1.04,
+// 750 nodes 1.12, 1.04, 1800 nodes 2.35, 1.40; 43 RVEs of 750 nodes 1.12, 1.50;
+// 128 RVEs of 200 nodes 1.72, 1.59 and 256 of them 2.60, 3.02.  Linear RVEs
+// beyond two nodes per thread pay for a third slot however little it holds, and
+// one direction's second round of workgroups is cheaper: with at most a quarter
+// of the slot in use up to two rounds (1760 nodes: 65 RVEs 2.54, 2.35, 85 RVEs
+// 2.71, 2.61; 1900 nodes 2.44, 2.40 and 2.56, 2.58), else up to one and a half (64
+// of 1950 nodes 2.38, 2.36; 65 of 2100 nodes 2.39, 2.50; toe law, 64 of 1800
+// nodes: 2.63, 2.75).  The largest RVE decides for all of them: workgroups of
+// three directions that start behind a round of one direction end last (85 RVEs
+// of 1850 nodes 3.3 instead of 2.5).
 void make_plan_tl(mf_batch *b) {
   int nv = 0;
   const Variant *vs = variants(&nv);
   b->plan_tl.assign(b->R, -1);
   b->lds_tl.assign(b->R, 0);
+  int top = 0;
+  for (const PackedRVE &p : b->host) top = std::max(top, p.Nf);
   for (int r = 0; r < b->R; ++r) {
     const PackedRVE &p = b->host[r];
-    const long room = p.Nf <= 256                       ? 3L * b->cus
-                      : p.Nf > 2 * 768 && all_linear(p) ? 3L * b->cus / 2
-                                                        : b->cus;
+    long room = b->cus;
+    if (p.Nf <= 256)
+      room = 3L * b->cus;
+    else if (p.Nf > 2 * 768 && all_linear(p))
+      room = top <= 2 * 768 + 768 / 4 ? 2L * b->cus : 3L * b->cus / 2;
     const bool spread = 6L * b->R <= room;
     long best_key = 0;
     for (int i = 0; i < nv; ++i) {
