@@ -285,7 +285,8 @@ int mf_batch_rve_sizes(const mf_batch *b, int32_t *sizes);
  * FP64 with the state in global memory (RVEs no other variant holds, in
  * either precision), 16384
  * FP64 evaluating each fiber once (bitwise the node-centric FP64 result),
- * 65536 FP64 for RVEs whose force records do not fit LDS (same result);
+ * 65536 FP64 for RVEs whose force records do not fit LDS, or whose fibers the
+ * registers of a forced thread count (same result);
  * bits 24-28: step chunks per solve of run() when more than one
  * (params.chunks).
  * Returns the number of distinct launch groups. */

@@ -459,11 +459,11 @@ int make_plan(mf_batch *b, int prec) {
       const long wave_rank = lin ? (v.block == 256 ? 0 : 10) : (v.block == 64 ? 0 : 10);
       const bool widen = wide > 0 && regs && !wave && v.npt == 1 &&
                          (wide == 768 ? v.block >= 512 && v.block <= 768 : v.block == wide);
-      // global-state FP64 last: only where nothing else fits.  FP64 with each
-      // fiber evaluated once before the node-centric FP64 kernels for RVEs
-      // with toe-law fibers (11% on 1500-node RVEs), after them for linear
-      // ones, whose cheap force does not pay for the extra phase (13% slower
-      // on 500-node RVEs)
+      // FP64: each fiber once from registers (1024 linear RVEs of 500 nodes 4.4
+      // ms, 10.3 with the IEEE kernels); then t records, widest workgroup first
+      // (their lists stream, and waves hide it); then node-centric without range
+      // handling; then the IEEE kernels, which energy diagnostics and RVEs
+      // outside fast64 run; the global state where nothing else fits
       long key = (v.flags & kGlobalState) ? 2000000000L
                  : (v.flags & kFast64)
                      ? ((v.flags & kFiberOnce) ? 600000000L : 700000000L) +
@@ -677,8 +677,9 @@ int64_t group_gstride(const Variant &v, int N) {
 // predecessor has finished long before it starts.  Each extra chunk costs its
 // solve a start and a state round trip, the time of 60-100 steps (4096 solves
 // of 500 nodes, 100 steps: 0.89, 1.40, 1.97, 2.65 ms in 1 to 4 chunks), and at
-// least 1%: three chunks give 6% at 3000 steps and take 36% at 300.  params.chunks > 0 forces the count, else the
-// autotuner's measured count when it set one.
+// least 1%: three chunks give 6% at 3000 steps and take 36% at 300.
+// params.chunks > 0 forces the count, else the autotuner's measured count when
+// it set one.
 int plan_chunks(const mf_batch *b, const Variant &v, size_t lds, int n) {
   if (b->p.mode != MF_MODE_RAMP || v.prec != MF_PREC_FP32C || !(v.flags & kEllInRegs) ||
       (v.flags & kWaveRve))

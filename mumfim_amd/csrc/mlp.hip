@@ -226,10 +226,11 @@ __global__ void ones_row_kernel(uint16_t *T, int64_t member_stride, int one_row,
 // silu'(z) of the same (sample, feature), which sits in the same lane.  G
 // members are evaluated at a time, eight waves each, and added in order.
 //
-// What bounds it: the activations' VALU work (2^20 samples, four members:
-// 1.0 ms of 1.4 ms) and, with J, the matrix cores (0.55 ms) and the weights'
-// way through L2 (280 KB per tile and member).  Measured on 2^20 samples /
-// 150001 with J: 2.73 / 2.31 ms with weights row by row, four waves of 64
+// What bounds it: the activations' VALU work (2^20 samples, four members: 0.74 of
+// the SIMD cycles, with the matrix cores at 0.39 and LDS at 0.54 beside it) and,
+// with J, the LDS reads of the activations (0.78, half of it bank conflicts), then
+// the matrix cores (0.57).  The weights come through L2, 280 KB per tile and
+// member.  Measured on 2^20 samples / 150001 with J: 2.73 / 2.31 ms with weights row by row, four waves of 64
 // features and accumulators in AGPRs (two or three waves per SIMD, each value
 // copied back before use); 2.39 / 1.49 ms with eight waves of 32 features (four
 // waves per SIMD, no copies, weights one k step ahead); 1.39 / 1.03 ms with

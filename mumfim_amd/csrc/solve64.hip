@@ -12,8 +12,6 @@ namespace kern {
 __device__ inline void sqrt64(double x, double &l, double &rl) {
   root64(x, __builtin_amdgcn_rsq(x), l, rl);
 }
-// Force of a nonlinear fiber (react64 with the stretch lr, g = (lr^2 - 1)/2
-// and 1/l0 at hand): both extensions are one formula with selected constants.
 typedef __attribute__((address_space(4))) Law64 law_const;
 // Three doubles per item in LDS as one 16-byte (x, y) array and one 8-byte z
 // array: gathering random items takes 20 CU cycles a wave (in-order ones 8),
@@ -35,6 +33,8 @@ struct Lds3 {
     *reinterpret_cast<lds_double *>((uintptr_t)(z + 8u * i)) = v[2];
   }
 };
+// Force of a nonlinear fiber (react64 with the stretch lr, g = (lr^2 - 1)/2
+// and 1/l0 at hand): both extensions are one formula with selected constants.
 __device__ inline double nonlinear64(const law_const &q, double lr, double g, double l0,
                                      double rl0) {
 #pragma clang fp contract(off)
@@ -226,11 +226,13 @@ __device__ __forceinline__ void finalize64(const SolveArgs &a, const RveDev &R, 
 // records in its ELL order, subtracting at end a and adding at end b, which
 // are solve64's roundings (an FMA by +-1 rounds as the addition does).
 //
-// What bounds it: FP64 instruction issue, then LDS.  So nothing that does not
-// change is computed or loaded in the step loop: a lane keeps its FPL fibers
+// What bounds it: FP64 instruction issue and LDS in turn, between two barriers
+// (0.66 of the SIMD cycles and 0.63 of the LDS cycles on 1024 RVEs of 500
+// nodes, 0.27 of the latter bank conflicts of the gathers).  So nothing that does
+// not change is computed or loaded in the step loop: a lane keeps its FPL fibers
 // (both ends' ranks, l0, 1/l0) and its nodes' first record references
 // (16 bits each) in registers, reaction constants are formed once
-// per solve, quotients by l0, m and l multiply by a reciprocal and correct
+// per batch, quotients by l0, m and l multiply by a reciprocal and correct
 // the result (div64), the two half kicks of a step share their quotient
 // except after a refresh, and the shortest fiber is a by-product of the
 // fiber phase.  Positions need one buffer: the node phase reads records only.
@@ -708,7 +710,8 @@ void solve64n(SolveArgs a) {
 // ============================================================================
 // FP64 fiber-once kernel for large RVEs
 // ============================================================================
-// solve64f's results for RVEs whose force records do not fit LDS.  Records
+// solve64f's results for RVEs whose force records do not fit LDS, or whose
+// fibers the registers of a forced thread count.  Records
 // hold t = f/l alone (8 bytes), and a node's gather recomputes d from the
 // positions, so these must stay until every gather is done: one buffer, and
 // the nodes drift in place after a barrier.  In RVEs with fibers of both laws
@@ -717,7 +720,7 @@ void solve64n(SolveArgs a) {
 // storage: a 4000-node RVE keeps 96 KB of positions and ~40 KB of records.
 // Fiber and list data stream from L2.  257 toe-law RVEs of 200-4000 nodes, 600
 // steps, whose largest RVEs end the batch: 11.8 ms, against 13.1 ms with the
-// node-centric kernel below, which evaluates every fiber twice, in waves of
+// node-centric kernel above, which evaluates every fiber twice, in waves of
 // mixed laws, and 20.4 ms with solve64.
 template <int B, int NPT>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4)))
