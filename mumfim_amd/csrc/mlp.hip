@@ -1173,14 +1173,11 @@ int mf_mlp_create(int32_t n_members, uint64_t seed, mf_mlp **out) {
     set_error("mf_mlp_create: stream/event creation failed");
     return fail(MF_ERR_HIP);
   }
-  static bool attr_done = false;
-  if (!attr_done) {
-    if (infer_attr<4, 0, 1>() != hipSuccess || infer_attr<1, 0, 2>() != hipSuccess ||
-        infer_attr<1, 6, 1>() != hipSuccess || infer_attr<1, 2, 2>() != hipSuccess) {
-      set_error("mf_mlp_create: LDS attribute");
-      return fail(MF_ERR_HIP);
-    }
-    attr_done = true;
+  // per device: the seven-plane tile needs 68 KB, above the 64 KB default
+  if (infer_attr<4, 0, 1>() != hipSuccess || infer_attr<1, 0, 2>() != hipSuccess ||
+      infer_attr<1, 6, 1>() != hipSuccess || infer_attr<1, 2, 2>() != hipSuccess) {
+    set_error("mf_mlp_create: LDS attribute");
+    return fail(MF_ERR_HIP);
   }
   const size_t K = n_members;
   std::vector<float> P(K * kNumParams);
