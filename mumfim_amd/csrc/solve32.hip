@@ -887,7 +887,7 @@ void solve32r(SolveArgs a) {
     double resid_local = 0.0;
 #pragma unroll
     for (int sl = 0; sl < NPT; ++sl)
-      if (own[sl]) node_force(sl, std::integral_constant<int, 0>{}, fint[sl], sl == 0);
+      if (own[sl]) node_force(sl, std::integral_constant<int, 0>{}, fint[sl], sl == 0 && wave_split);
     double lmin2 = min_length2(cur);
     red_min_sum(lmin2, resid_local);
     const float h = crit_half * (sqrtf((float)lmin2) * inv_c);
